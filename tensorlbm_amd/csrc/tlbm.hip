@@ -621,9 +621,27 @@ struct ZRing {
   static constexpr int ROWS = OFF_C + 4 * NC;  // 57 for D3Q19 (= 3 Q), 81 for D3Q27
 };
 
-// Two fused steps per launch (temporal blocking).  A workgroup owns a TX x TY
+// Launch shape of the two-step kernel: output tile tx x ty, z planes per workgroup,
+// and whether the stores bypass L2 (non-temporal).
+struct Plan2 {
+  int tx, ty, zc, nt;
+};
+
+// Tile cells (halo included) a two-step workgroup has LDS rows for: 66 x 10 where
+// the ring fits the 160 KB of LDS next to the mask and f_eq tables, else 34 x 10
+// (D3Q27 with 4-byte storage).  Lanes: one per tile cell, rounded to whole waves.
+template <class L, int S>
+constexpr int tile2_cells() {
+  return 3 * L::Q * 66 * 10 * int(sizeof(typename Store<S>::T)) <= 158 * 1024 ? 66 * 10 : 34 * 10;
+}
+template <class L, int S>
+constexpr int tile2_threads() {
+  return (tile2_cells<L, S>() + 63) / 64 * 64;
+}
+
+// Two fused steps per launch (temporal blocking).  A workgroup owns a tx x ty
 // column of output cells and marches z over `zc` planes.  Step-one states of a
-// (TX+2) x (TY+2) tile (one cell per lane, read from HBM) are kept in LDS for
+// (tx+2) x (ty+2) tile (one cell per lane, read from HBM) are kept in LDS for
 // three consecutive planes, in the storage format, so step two sees exactly the
 // values a second launch would read; step two pulls from LDS, so a cell's
 // populations cross HBM once per two steps plus the tile halo.  The step-one
@@ -633,13 +651,18 @@ struct ZRing {
 // the solid cells are the five stationary walls of a cubic lid-driven cavity
 // (x = 0, x = nx-1, y = 0, z = 0, z = nz-1), decided from the coordinates
 // instead of read from a mask.
-template <class L, int S, int COLL, int FEAT, int BCK, int TX, int TY, bool BoxWalls = false>
-__device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, int zc, uint32_t tile) {
+template <class L, int S, int COLL, int FEAT, int BCK, bool BoxWalls = false>
+__device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, const Plan2& p2, uint32_t tile) {
   using ST = Store<S>;
   using T = typename ST::T;
   using C = typename ST::C;
   constexpr int Q = L::Q;
-  constexpr int EX = TX + 2, EY = TY + 2, EC = EX * EY;
+  constexpr int EC = tile2_cells<L, S>();
+  // The tile is a launch parameter: 64 x 8 where rows are whole cache lines, else the
+  // shape that wastes fewest lanes on this grid (plan2).  The LDS rows keep a fixed
+  // pitch of EC cells, so a run-time tile costs three more address registers than a
+  // compile-time one and nothing in the plane loop (256^3 channel: 480 us either way).
+  const int TX = p2.tx, TY = p2.ty, zc = p2.zc, EX = TX + 2;
   constexpr bool kAll = (FEAT & FEAT_BC) != 0;
   constexpr bool kForce = (FEAT & FEAT_FORCE) != 0;
   static_assert((FEAT & FEAT_MLP) == 0, "the closure runs in the one-step kernel");
@@ -663,7 +686,7 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
   const int zend = z0 + zc < nz ? z0 + zc : nz;
   const T* fin = static_cast<const T*>(a.fin);
   // step-one cell of this lane (tile-local lx, ly; global gx, gy)
-  const bool h1 = t < EC;
+  const bool h1 = t < EX * (TY + 2);
   const int lx = h1 ? t % EX : 0, ly = h1 ? t / EX : 0;
   const int gx0 = x0 - 1 + lx, gy0 = y0 - 1 + ly;
   const int gx = (gx0 % nx + nx) % nx;  // halo lanes of a tile wider than the lattice wrap more than once
@@ -682,11 +705,12 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
   // instead and compute it from the same inputs with the same code, so every
   // wave runs the update unmasked; only lanes that own their cell store (`own`),
   // so no cell is written twice.
-  static_assert(TX * TY % 64 == 0, "output lanes fill whole waves");
   const bool out_wave = __builtin_amdgcn_readfirstlane(t) < TX * TY;
   const bool h2 = t < TX * TY;
   const int ux_ = min(x0 + (h2 ? t % TX : 0), nx - 1), uy_ = min(y0 + (h2 ? t / TX : 0), ny - 1);
   const int ox = ux_ - x0, oy = uy_ - y0;
+  // tile cells of this lane's pulls by c_y (0, +1, -1), shifted by -c_x at the use
+  const int at_0 = (oy + 1) * EX + ox + 1, at_p = at_0 - EX, at_m = at_0 + EX;
   const bool own = h2 && x0 + t % TX < nx && y0 + t / TX < ny;
   double unused_force = 0.0;
   // Ladd force of both steps (obstacles.py:91-130), each cell of the launch's output range
@@ -795,17 +819,17 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
       // plane only: the boundary overrides read along x), written as plane
       // k + 1 - c_z[q] of the march
       const int row_a = set_row(-1, k + 2), row_b = set_row(0, k + 1), row_c = set_row(1, k);
-      auto lds_at = [&](int q, int x, int y, int) -> C {
+      auto lds_at = [&](int q, int x, int, int) -> C {  // only ever for this lane's y
         const int row = (L::cz[q] < 0 ? row_a : L::cz[q] == 0 ? row_b : row_c) + R::index(q);
-        const int sx = x - L::cx[q] - (x0 - 1), sy = y - L::cy[q] - (y0 - 1);
-        return ST::template get<L>(s[row * EC + sy * EX + sx], q);
+        const int at = L::cy[q] == 0 ? at_0 : (L::cy[q] > 0 ? at_p : at_m);
+        return ST::template get<L>(s[row * EC + at + (x - ux_) - L::cx[q]], q);
       };
       C f[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q) f[q] = lds_at(q, ux_, uy_, z);
       const uint32_t cell = (uint32_t(z) * uint32_t(ny) + uint32_t(uy_)) * uint32_t(nx) + uint32_t(ux_);
       bool solid = false;
-      if constexpr (kAll) solid = s_solid[((k + 1) % 3) * EC + (oy + 1) * EX + (ox + 1)] != 0;
+      if constexpr (kAll) solid = s_solid[((k + 1) % 3) * EC + at_0] != 0;
       if constexpr (kForce) {
         double sx = 0.0, sy = 0.0, sz = 0.0;
         update_cell<L, S, COLL, true, FEAT, BCN_PULL, BCK>(f, a, ux_, uy_, z, cell, solid, false, sx, sy, sz, lds_at,
@@ -822,16 +846,21 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
       }
       T* fout = static_cast<T*>(a.fout);
       const uint32_t off = uint32_t(uy_) * uint32_t(a.osy) + uint32_t(ux_);
-      // cavity rows (pitch = edge) rarely start on a cache line, and non-temporal
-      // stores of the partial lines at a tile's ends each reach HBM: on 64
-      // cavities of edges 32-160 that wrote 1.21x the least bytes and ran at 42.1
-      // GLUPS; through L2, 1.02x and 48.6 GLUPS
-      if (own) {
+      // Rounded before the choice of store: folded into the two store loops the last
+      // operations of the update would be contracted differently from the one-step kernel.
+      T o[Q];
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-          T* const base = fout + int64_t(q) * a.osq + int64_t(z) * a.osz;
-          if constexpr (BoxWalls) st_l2(base, off, put_out<L, S, COLL>(f[q], q));
-          else st_nt(base, off, put_out<L, S, COLL>(f[q], q));
+      for (int q = 0; q < Q; ++q) {
+        o[q] = put_out<L, S, COLL>(f[q], q);
+        asm volatile("" : "+v"(o[q]));
+      }
+      if (own) {
+        if (p2.nt) {
+#pragma unroll
+          for (int q = 0; q < Q; ++q) st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, o[q]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < Q; ++q) st_l2(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, o[q]);
         }
       }
     } else {
@@ -848,15 +877,10 @@ __global__ __launch_bounds__(256) void k_lbm(const KArgs<typename Store<S>::C> a
   lbm_body<L, S, COLL, STREAM, FEAT, BCK>(a);
 }
 
-// two-step tile: TX x TY output cells, (TX+2)(TY+2) lanes rounded to whole waves
-template <int TX, int TY>
-constexpr int tb_threads() {
-  return ((TX + 2) * (TY + 2) + 63) / 64 * 64;
-}
-
-template <class L, int S, int COLL, int FEAT, int BCK, int TX, int TY>
-__global__ __launch_bounds__((tb_threads<TX, TY>())) void k_lbm2(const KArgs<typename Store<S>::C> a, int zc) {
-  lbm2_body<L, S, COLL, FEAT, BCK, TX, TY>(a, zc, xcd_tile(blockIdx.x, gridDim.x));
+template <class L, int S, int COLL, int FEAT, int BCK>
+__global__ __launch_bounds__((tile2_threads<L, S>())) void k_lbm2(const KArgs<typename Store<S>::C> a,
+                                                                  const Plan2 p2) {
+  lbm2_body<L, S, COLL, FEAT, BCK>(a, p2, xcd_tile(blockIdx.x, gridDim.x));
 }
 
 // The learned-closure step.  Its collision is long (the network runs on the
@@ -1562,21 +1586,13 @@ int launch_lbm_kind(const KArgs<typename Store<S>::C>& a, int bx, int by, uint32
 
 // ---- two steps per launch ----------------------------------------------------
 
-// Tile of the two-step kernel: 64 x 8 output cells (11 waves, 1.29x halo reads;
-// D3Q19 fp32: 150 KB for three planes) where three planes fit the 160 KB of LDS
-// next to the mask and f_eq tables, else 32 x 8 (6 waves; D3Q27 with 4-byte
-// storage).  Measured on the 256^3 channel: 64 x 6 46.0, 64 x 7 50.7, 64 x 8
-// 57.2 GLUPS (more waves per CU and less recomputed halo).  32 x 16 recomputes
-// less halo (1.20x against 1.29x) and pads uneven grids less, yet ran slower:
-// 61.6 against 64.9 GLUPS on the channel and 34.6 against 42.2 on 64 cavities
-// of edges 32-160 -- rows of 64 keep each pulled row in whole cache lines.
-template <class L, int S>
-struct Tile2 {
-  static constexpr bool wide = 3 * L::Q * 66 * 10 * sizeof(typename Store<S>::T) <= 158 * 1024;
-  static constexpr int TX = wide ? 64 : 32;
-  static constexpr int TY = 8;
-};
-
+// Base tile of the two-step kernel: 64 x 8 output cells (11 waves, 1.29x halo reads)
+// where the LDS rows allow it, else 32 x 8 (6 waves; D3Q27 with 4-byte storage).
+// Measured on the 256^3 channel: 64 x 6 46.0, 64 x 7 50.7, 64 x 8 57.2 GLUPS (more
+// waves per CU and less recomputed halo); 32 x 16 recomputes less halo (1.20x) but ran
+// slower (518 against 480 us per launch): rows of 64 keep each pulled row in whole
+// cache lines.  Two half-size workgroups per CU (34 x 10 cells each, at most 128 VGPRs)
+// took 664-678 us.
 inline int tile2_width(int lattice, int store) {
   return lattice == TLBM_D3Q27 && store == TLBM_STORE_F32 ? 32 : 64;
 }
@@ -1599,25 +1615,89 @@ inline int device_cus() {
   return v;
 }
 
-// z planes per workgroup.  A two-step workgroup holds most of a CU's LDS, so a CU
+// Launch shape of the two-step kernel.  A workgroup holds most of a CU's LDS, so a CU
 // runs one at a time and a launch of W = cols * ceil(nz / zc) workgroups takes
-// ceil(W / CUs) rounds of about zc + 2 plane times (zc planes, the two-plane fill
-// of the march at half cost, the prologue).  Pick the zc with the least total:
-// on MI355X at 256^3 that is 128 (one round of 256 workgroups; 60.7 GLUPS on the
-// channel + sphere against 59.1 / 57.2 / 54.8 for zc = 64 / 32 / 16, whose
-// costs this model ranks and spaces the same way).
-inline int step2_zc(int cols, int nz, int cus) {
+// ceil(W / CUs) rounds of about zc + 2 plane times (zc planes, the two-plane fill of
+// the march at half cost, the prologue).  zc_of returns the zc with the least
+// rounds * (zc + 2) and that cost: on MI355X at 256^3 that is 128 (one round of 256
+// workgroups; 60.7 GLUPS on the channel + sphere against 59.1 / 57.2 / 54.8 for
+// zc = 64 / 32 / 16, whose costs this model ranks and spaces the same way).  For a
+// number of rounds r the best chunk count is the largest that fits, r * CUs / cols.
+inline int zc_of(int64_t cols, int nz, int cus, int64_t* cost) {
   int best = nz;
   int64_t best_cost = INT64_MAX;
-  for (int zc = 1; zc <= nz; ++zc) {
-    const int64_t w = int64_t(cols) * ((nz + zc - 1) / zc);
-    const int64_t cost = (w + cus - 1) / cus * (zc + 2);
-    if (cost < best_cost) {
-      best_cost = cost;
+  for (int64_t r = (cols + cus - 1) / cus; 2 * r + cols * nz / cus < best_cost; ++r) {
+    const int64_t k = r * cus / cols;  // >= 1
+    const int zc = k >= nz ? 1 : int((nz + k - 1) / k);
+    const int64_t c = (cols * ((nz + zc - 1) / zc) + cus - 1) / cus * (zc + 2);
+    if (c < best_cost) {
+      best_cost = c;
       best = zc;
     }
+    if (k >= nz) break;
   }
+  if (cost) *cost = best_cost;
   return best;
+}
+
+// Relative time of a launch with output tiles tx x ty on an (ny, nx) plane: rounds *
+// (zc + 2) plane times, a plane time growing with the waves of both steps and with the
+// cache lines its pulled rows touch (a tile as wide as the grid reads contiguously).
+// Fitted to 630 timed launches on 61 grids; picks within 3 % of the best shape tried
+// on average.
+inline double tile2_cost(int tx, int ty, int ny, int nx, int nz, int esize, int cus, int* zc) {
+  const int64_t cols = int64_t((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
+  int64_t c;
+  *zc = zc_of(cols, nz, cus, &c);
+  const int w = ((tx + 2) * (ty + 2) + 63) / 64 + (tx * ty + 63) / 64;
+  const double lines = (ty + 2) * ((tx + 2) * esize / 128.0 + (tx == nx ? 0.2 : 1.0));
+  return double(c) * (8 + w + 0.1 * lines);
+}
+
+// The output tile of a D3Q19 grid whose rows are not whole cache lines, and how its
+// results are stored.  Candidates: the base tile; the full row (up to 108 cells: at
+// least four rows of it fit), whose lanes then read and write contiguous memory; and
+// from nx = 128 the row cut into floor(nx / 64) equal parts, wider than 64.
+// Measured on 61 grids of 20-256 cells an edge, fp32 BGK / MRT and fp16-deviation BGK,
+// against 64 x 8 with non-temporal stores throughout (the shape before): 1.07x on
+// average, 0.98x-1.6x; e.g. (245, 185, 68) 143 -> 106 us, MRT 185 -> 119 us;
+// (131, 147, 211) MRT 199 -> 172 us.
+//
+// Stores: non-temporal where rows or whole tiles are contiguous lines (through L2 they
+// took 3-11 % longer).  Otherwise a tile's rows end in partial lines that only merge
+// with the neighbouring tile's in L2: through L2 is up to 1.4x faster, except where
+// one lattice takes 120-256 MB.  There the input still sits in the 256 MB last-level
+// cache, stores through L2 push it out (0.8x), and narrower tiles lose as well.
+inline Plan2 plan2(int ny, int nx, int nz, int64_t pitch, int esize, int cells, bool outlet, int cus) {
+  const auto rows = [&](int tx) {
+    int ty = cells / (tx + 2) - 2;
+    if (ty > ny) ty = ny;
+    const int nty = (ny + ty - 1) / ty;
+    return (ny + nty - 1) / nty;
+  };
+  Plan2 s{64, 8, 1, 1};
+  double best = tile2_cost(64, 8, ny, nx, nz, esize, cus, &s.zc);
+  const bool aligned = pitch * esize % 128 == 0;
+  if (aligned && nx % 64 == 0) return s;
+  const double mb = 1e-6 * 19 * esize * double(nz) * ny * nx;
+  const bool cached = mb > 120.0 && mb <= 256.0;
+  s.nt = aligned || cached || mb < 45.0;
+  const auto consider = [&](int tx, double bias, int nt) {
+    if (outlet && (nx < 4 || (nx - 1) % tx < 2)) return;  // as step2_reason for the base tile
+    const int ty = rows(tx);
+    int zc;
+    const double c = bias * tile2_cost(tx, ty, ny, nx, nz, esize, cus, &zc);
+    if (c < best) {
+      best = c;
+      s = Plan2{tx, ty, zc, nt};
+    }
+  };
+  if (nx >= 16 && nx <= 108) consider(nx, 1.0, pitch == nx);
+  if (!aligned && !cached && nx > 128) {
+    const int parts = nx / 64;
+    consider((nx + parts - 1) / parts, 1.05, 0);
+  }
+  return s;
 }
 
 // Batched lid-driven cavities, two steps per launch: the two-step march over the
@@ -1631,7 +1711,8 @@ inline int step2_zc(int cols, int nz, int cus) {
 struct Cav2Dev {
   int64_t offset;
   uint32_t tiles_before;
-  int32_t edge;
+  uint16_t edge;
+  uint8_t tx, ty;  // output tile of this cavity
   double omega;
 };
 
@@ -1645,7 +1726,7 @@ struct Cav2Args {
 static_assert(sizeof(Cav2Args<float>) < 4000, "cavity table travels in the kernel arguments");
 
 template <int S>
-__global__ __launch_bounds__((tb_threads<Tile2<D3Q19, S>::TX, Tile2<D3Q19, S>::TY>())) void k_cav2(
+__global__ __launch_bounds__((tile2_threads<D3Q19, S>())) void k_cav2(
     const Cav2Args<typename Store<S>::C> a) {
   using T = typename Store<S>::T;
   using C = typename Store<S>::C;
@@ -1666,41 +1747,53 @@ __global__ __launch_bounds__((tb_threads<Tile2<D3Q19, S>::TX, Tile2<D3Q19, S>::T
   k.isy = k.osy = E;
   k.omega = C(a.c[lo].omega);
   k.tau = C(1.0 / a.c[lo].omega);
-  lbm2_body<D3Q19, S, TLBM_COLL_BGK, FEAT_BC, TLBM_BC_LID_Y, Tile2<D3Q19, S>::TX, Tile2<D3Q19, S>::TY, true>(
-      k, a.zc, g - a.c[lo].tiles_before);
+  const Plan2 p2{a.c[lo].tx, a.c[lo].ty, a.zc, 0};
+  lbm2_body<D3Q19, S, TLBM_COLL_BGK, FEAT_BC, TLBM_BC_LID_Y, true>(k, p2, g - a.c[lo].tiles_before);
 }
 
-// Workgroups of a two-step cavity launch with z chunks of zc planes, per cavity
-// prefix sums into `a`; -1 when the count would not fit 31 bits.
-template <typename C, int TX, int TY>
-int64_t cav2_layout(Cav2Args<C>& a, const tlbm_cavity* cavs, int n, int zc) {
-  uint64_t w = 0;
-  for (int i = 0; i < n; ++i) {
-    const int E = int(cavs[i].edge);
-    a.c[i].offset = cavs[i].offset;
-    a.c[i].tiles_before = uint32_t(w);
-    a.c[i].edge = E;
-    a.c[i].omega = 1.0 / cavs[i].tau;
-    w += uint64_t((E + TX - 1) / TX) * uint64_t((E + TY - 1) / TY) * uint64_t((E + zc - 1) / zc);
-    if (w >= (uint64_t(1) << 31)) return -1;
+// Output tile of a cavity of edge E: the base tile, the full row or the row in equal
+// parts wider than 64 (the candidates of plan2), whichever costs the batch least
+// plane time (the number of columns times a column's plane time; the z chunk is
+// common to the batch).
+template <class L, int S>
+void cav2_tile(int E, uint8_t* tx, uint8_t* ty) {
+  constexpr int cells = tile2_cells<L, S>();
+  constexpr double esize = sizeof(typename Store<S>::T);
+  double best = 1e300;
+  const int parts = E / 64 > 0 ? E / 64 : 1;
+  const int cand[3] = {64, E <= 108 ? E : 64, E > 128 && E < 65536 ? (E + parts - 1) / parts : 64};
+  for (int i = 0; i < 3; ++i) {
+    const int w = cand[i];
+    int h = i == 0 || w == 64 ? 8 : cells / (w + 2) - 2;
+    if (h > E) h = E;
+    const int rows = (E + h - 1) / h;
+    h = (E + rows - 1) / rows;
+    const int waves = ((w + 2) * (h + 2) + 63) / 64 + (w * h + 63) / 64;
+    const double lines = (h + 2) * ((w + 2) * esize / 128.0 + (w == E ? 0.2 : 1.0));
+    const double c = double((E + w - 1) / w) * rows * (8 + waves + 0.1 * lines) * (i == 2 ? 1.05 : 1.0);
+    if (c < best) {
+      best = c;
+      *tx = uint8_t(w);
+      *ty = uint8_t(h);
+    }
   }
-  return int64_t(w);
+}
+
+inline int64_t cav2_cols(const Cav2Dev& c) {
+  return int64_t((c.edge + c.tx - 1) / c.tx) * ((c.edge + c.ty - 1) / c.ty);
 }
 
 // z planes per workgroup for a batch of cavities: the rounds x planes model of
-// step2_zc over the workgroups of all cavities together
-template <int TX, int TY>
-int cav2_zc(const tlbm_cavity* cavs, int n, int cus) {
+// zc_of over the workgroups of all cavities together
+template <typename C>
+int cav2_zc(const Cav2Args<C>& a, int cus) {
   int emax = 1;
-  for (int i = 0; i < n; ++i) emax = cavs[i].edge > emax ? int(cavs[i].edge) : emax;
+  for (int i = 0; i < a.n; ++i) emax = a.c[i].edge > emax ? int(a.c[i].edge) : emax;
   int best = emax;
   int64_t best_cost = INT64_MAX;
   for (int zc = 1; zc <= emax; ++zc) {
     int64_t w = 0;
-    for (int i = 0; i < n; ++i) {
-      const int E = int(cavs[i].edge);
-      w += int64_t((E + TX - 1) / TX) * ((E + TY - 1) / TY) * ((E + zc - 1) / zc);
-    }
+    for (int i = 0; i < a.n; ++i) w += cav2_cols(a.c[i]) * ((a.c[i].edge + zc - 1) / zc);
     const int64_t cost = (w + cus - 1) / cus * (zc + 2);
     if (cost < best_cost) {
       best_cost = cost;
@@ -1713,7 +1806,6 @@ int cav2_zc(const tlbm_cavity* cavs, int n, int cus) {
 template <int S>
 int launch_cav2(const void* fin, void* fout, const tlbm_cavity* cavs, int n, double u_lid, int zc, hipStream_t s) {
   using C = typename Store<S>::C;
-  constexpr int TX = Tile2<D3Q19, S>::TX, TY = Tile2<D3Q19, S>::TY;
   Cav2Args<C> a;
   memset(&a, 0, sizeof(a));
   a.k.fin = fin;
@@ -1723,11 +1815,22 @@ int launch_cav2(const void* fin, void* fout, const tlbm_cavity* cavs, int n, dou
   a.k.bc_kind = TLBM_BC_LID_Y;
   a.k.bc_u[0] = C(u_lid);
   a.n = n;
-  a.zc = zc > 0 ? zc : cav2_zc<TX, TY>(cavs, n, device_cus());
-  const int64_t w = cav2_layout<C, TX, TY>(a, cavs, n, a.zc);
-  if (w < 0) return fail(TLBM_ERR_SHAPE, "too many workgroups for one launch");
+  for (int i = 0; i < n; ++i) {
+    a.c[i].offset = cavs[i].offset;
+    a.c[i].edge = uint16_t(cavs[i].edge);
+    a.c[i].omega = 1.0 / cavs[i].tau;
+    cav2_tile<D3Q19, S>(int(cavs[i].edge), &a.c[i].tx, &a.c[i].ty);
+  }
+  a.zc = zc > 0 ? zc : cav2_zc(a, device_cus());
+  // workgroups of the launch, as per-cavity prefix sums
+  uint64_t w = 0;
+  for (int i = 0; i < n; ++i) {
+    a.c[i].tiles_before = uint32_t(w);
+    w += uint64_t(cav2_cols(a.c[i])) * uint64_t((a.c[i].edge + a.zc - 1) / a.zc);
+    if (w >= (uint64_t(1) << 31)) return fail(TLBM_ERR_SHAPE, "too many workgroups for one launch");
+  }
   a.total = uint32_t(w);
-  hipLaunchKernelGGL(k_cav2<S>, dim3(a.total), dim3(tb_threads<TX, TY>()), 0, s, a);
+  hipLaunchKernelGGL(k_cav2<S>, dim3(a.total), dim3(tile2_threads<D3Q19, S>()), 0, s, a);
   return check_launch("k_cav2");
 }
 
@@ -1749,11 +1852,21 @@ inline const char* step2_reason(int lattice, int store, const tlbm_collision* co
 
 template <class L, int S, int COLL, int FEAT, int BCK>
 int launch_lbm2(const KArgs<typename Store<S>::C>& a, hipStream_t s) {
-  constexpr int TX = Tile2<L, S>::TX, TY = Tile2<L, S>::TY;
-  const int gx = (a.nx + TX - 1) / TX, gy = (a.ny + TY - 1) / TY;
-  const int zc = step2_zc(gx * gy, a.nz, device_cus());
-  const uint32_t tiles = uint32_t(gx) * uint32_t(gy) * uint32_t((a.nz + zc - 1) / zc);
-  hipLaunchKernelGGL((k_lbm2<L, S, COLL, FEAT, BCK, TX, TY>), dim3(tiles), dim3(tb_threads<TX, TY>()), 0, s, a, zc);
+  constexpr int cells = tile2_cells<L, S>(), esize = sizeof(typename Store<S>::T);
+  constexpr int width = cells == 66 * 10 ? 64 : 32;
+  Plan2 p{width, 8, 1, 1};
+  if constexpr (L::Q == 19) {
+    const bool outlet = a.bc_kind == TLBM_BC_CHANNEL_X || a.bc_kind == TLBM_BC_FAR_FIELD;
+    p = plan2(a.ny, a.nx, a.nz, a.osy, esize, cells, outlet, device_cus());
+  } else {
+    const int64_t cols = int64_t((a.nx + width - 1) / width) * ((a.ny + 7) / 8);
+    p.zc = zc_of(cols, a.nz, device_cus(), nullptr);
+  }
+  const uint64_t tiles = uint64_t((a.nx + p.tx - 1) / p.tx) * uint64_t((a.ny + p.ty - 1) / p.ty) *
+                         uint64_t((a.nz + p.zc - 1) / p.zc);
+  if (tiles >= (uint64_t(1) << 31)) return fail(TLBM_ERR_SHAPE, "too many workgroups");
+  hipLaunchKernelGGL((k_lbm2<L, S, COLL, FEAT, BCK>), dim3(uint32_t(tiles)), dim3(tile2_threads<L, S>()), 0, s, a,
+                     p);
   return check_launch("k_lbm2");
 }
 
