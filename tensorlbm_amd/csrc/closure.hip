@@ -81,159 +81,288 @@ __global__ __launch_bounds__(64) void k_mlp_pack(const float* __restrict__ p, Pa
 // fp32 forward (prediction) and gradient
 // ---------------------------------------------------------------------------
 
-struct Fwd {
-  float xh[NIN], z1[NH], z2[NH], z3, y;
-};
-
-__device__ __forceinline__ void forward32(const float* __restrict__ p, const float* x, Fwd& r) {
-#pragma unroll
-  for (int e = 0; e < NIN; ++e) r.xh[e] = (x[e] - p[OMEAN + e]) * p[OISTD + e];
-  for (int i = 0; i < NH; ++i) {
-    float a = p[OB1 + i];
-#pragma unroll
-    for (int e = 0; e < NIN; ++e) a += p[OW1 + i * NIN + e] * r.xh[e];
-    r.z1[i] = a;
-  }
-  for (int i = 0; i < NH; ++i) {
-    float a = p[OB2 + i];
-    for (int j = 0; j < NH; ++j) a += p[OW2 + i * NH + j] * fmaxf(r.z1[j], 0.0f);
-    r.z2[i] = a;
-  }
-  float a = p[OB3];
-  for (int i = 0; i < NH; ++i) a += p[OW3 + i] * fmaxf(r.z2[i], 0.0f);
-  r.z3 = a;
-  r.y = softplus(a);
-}
-
+// One lane per sample, the whole network unrolled: activations in registers, weights
+// by scalar loads (their index is uniform).  With rolled loops over a per-lane
+// activation array the array lived in scratch memory (13,107 samples: 17.4 us).
 __global__ __launch_bounds__(256) void k_mlp_predict(const float* __restrict__ p, const float* __restrict__ x,
                                                      uint64_t n, float* __restrict__ y) {
   const uint64_t s = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (s >= n) return;
-  float xs[NIN];
+  float xh[NIN], h1[NH];
 #pragma unroll
-  for (int e = 0; e < NIN; ++e) xs[e] = x[s * NIN + e];
-  Fwd r;
-  forward32(p, xs, r);
-  y[s] = r.y;
+  for (int e = 0; e < NIN; ++e) xh[e] = (x[s * NIN + e] - p[OMEAN + e]) * p[OISTD + e];
+#pragma unroll
+  for (int i = 0; i < NH; ++i) {
+    float a = p[OB1 + i];
+#pragma unroll
+    for (int e = 0; e < NIN; ++e) a += p[OW1 + i * NIN + e] * xh[e];
+    h1[i] = fmaxf(a, 0.0f);
+  }
+  float z3 = p[OB3];
+#pragma unroll 4
+  for (int i = 0; i < NH; ++i) {
+    float a = p[OB2 + i];
+#pragma unroll
+    for (int j = 0; j < NH; ++j) a += p[OW2 + i * NH + j] * h1[j];
+    z3 += p[OW3 + i] * fmaxf(a, 0.0f);
+  }
+  y[s] = softplus(z3);
 }
 
-// Each workgroup: 64 samples (one per lane of wave 0) run forward + backward,
-// park activations and deltas in LDS, then 256 lanes reduce the 1345 parameter
-// gradients (and the loss) over the 64 samples into partials[block].
+// Gradient of 64 samples per workgroup into partials[block].  Lane = sample, and each
+// of the four waves carries a quarter of the hidden units through the forward and the
+// backward pass, so that all four SIMDs of a CU work (with one wave running all units
+// and its activation arrays in scratch memory, 4096 samples took 25 us).  The parameters are
+// staged into LDS in one round of loads beside the sample's own (read where they are
+// used, by scalar loads, each layer waited for several round trips: 10 us); every lane
+// of a wave reads the same weight, an LDS broadcast.  Activations and deltas go
+// through LDS as [unit][sample].  The weight gradients are products
+// delta^T activation over the 64 samples: fp32 matrix-core tiles (16 x 16, exact fp32
+// products and accumulation), whose operands the LDS pitch of 68 floats serves without
+// bank conflicts (bank 4 unit + sample).
+//   A: lane -> row lane % 16, k = lane / 16;  B: column lane % 16, k = lane / 16;
+//   D: rows 4 (lane / 16) + r, column lane % 16.
+// idx (optional) names the rows of x and t to take, so a minibatch needs no copy.
+constexpr int GP = 68;  // LDS pitch of a unit's 64 samples
+static_assert(OW2 % 4 == 0 && NH % 4 == 0, "four weights of a row of W2 are 16-byte aligned in LDS");
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <class FA, class FB>
+__device__ __forceinline__ f32x4 grad_tile(int lane, const FA& a, const FB& b) {
+  f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int k = 0; k < GRAD_BS; k += 4) {
+    const int sm = k + (lane >> 4);
+    d = __builtin_amdgcn_mfma_f32_16x16x4f32(a(lane & 15, sm), b(lane & 15, sm), d, 0, 0, 0);
+  }
+  return d;
+}
+
+__device__ __forceinline__ float wave_sum64(float v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
 __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ p, const float* __restrict__ x,
-                                                  const float* __restrict__ t, uint64_t n, float inv_n,
-                                                  float* __restrict__ partials) {
-  __shared__ float s_xh[GRAD_BS][8];
-  __shared__ float s_h1[GRAD_BS][NH];
-  __shared__ float s_d1[GRAD_BS][NH];
-  __shared__ float s_h2[GRAD_BS][NH];
-  __shared__ float s_d2[GRAD_BS][NH];
-  __shared__ float s_d3[GRAD_BS];
-  __shared__ float s_loss[GRAD_BS];
-  const int tid = threadIdx.x;
-  if (tid < GRAD_BS) {
-    const uint64_t s = uint64_t(blockIdx.x) * GRAD_BS + tid;
-    const bool ok = s < n;
-    float xs[NIN];
+                                                  const float* __restrict__ t, const int64_t* __restrict__ idx,
+                                                  uint64_t n, float inv_n, float* __restrict__ partials) {
+  constexpr int U = NH / 4;  // hidden units per wave
+  __shared__ float s_xb[8][GP];  // normalised inputs, then a row of ones (the bias column)
+  __shared__ float s_h1[NH][GP], s_d1[NH][GP], s_h2[NH][GP], s_d2[NH][GP];
+  __shared__ float s_z3[4][GRAD_BS], s_d3[GRAD_BS];
+  __shared__ __align__(16) float s_p[(NTOTAL + 3) / 4 * 4];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int u0 = w * U;
+  const uint64_t s = uint64_t(blockIdx.x) * GRAD_BS + lane;
+  const bool ok = s < n;
+  const uint64_t row = ok ? (idx != nullptr ? uint64_t(idx[s]) : s) : 0;
+  float pv[(NTOTAL + 255) / 256];
 #pragma unroll
-    for (int e = 0; e < NIN; ++e) xs[e] = ok ? x[s * NIN + e] : 0.0f;
-    Fwd r;
-    forward32(p, xs, r);
-    const float res = ok ? r.y - t[s] : 0.0f;
-    s_loss[tid] = res * res * inv_n;
-    // dL/dz3 = 2 (y - t)/N * softplus'(z3): sigmoid(beta z3), 1 where softplus returns z3 (beta z3 > 20)
-    const float bz = fmaxf(BETA * r.z3, -60.0f);
-    const float d3 = 2.0f * res * inv_n * (bz > 20.0f ? 1.0f : 1.0f / (1.0f + __expf(-bz)));
-    s_d3[tid] = d3;
-    float d2[NH];
-    for (int i = 0; i < NH; ++i) {
-      d2[i] = r.z2[i] > 0.0f ? d3 * p[OW3 + i] : 0.0f;
-      s_d2[tid][i] = d2[i];
-      s_h2[tid][i] = fmaxf(r.z2[i], 0.0f);
-    }
-    for (int j = 0; j < NH; ++j) {
-      float a = 0.0f;
-      for (int i = 0; i < NH; ++i) a += d2[i] * p[OW2 + i * NH + j];
-      s_d1[tid][j] = r.z1[j] > 0.0f ? a : 0.0f;
-      s_h1[tid][j] = fmaxf(r.z1[j], 0.0f);
-    }
+  for (int k = 0; k < (NTOTAL + 255) / 256; ++k) {
+    const int i = int(threadIdx.x) + 256 * k;
+    pv[k] = i < NTOTAL ? p[i] : 0.0f;
+  }
+  const float target = ok ? t[row] : 0.0f;
+  float xh[NIN];
 #pragma unroll
-    for (int e = 0; e < NIN; ++e) s_xh[tid][e] = r.xh[e];
-    s_xh[tid][7] = 0.0f;
+  for (int e = 0; e < NIN; ++e) xh[e] = ok ? x[row * NIN + e] : 0.0f;
+#pragma unroll
+  for (int k = 0; k < (NTOTAL + 255) / 256; ++k) {
+    const int i = int(threadIdx.x) + 256 * k;
+    if (i < NTOTAL) s_p[i] = pv[k];
   }
   __syncthreads();
-  float* out = partials + uint64_t(blockIdx.x) * (NPARAM + 1);
-  for (int k = tid; k <= NPARAM; k += blockDim.x) {
-    float g = 0.0f;
-    if (k < OB1) {
-      const int i = k / NIN, e = k % NIN;
-      for (int s = 0; s < GRAD_BS; ++s) g += s_d1[s][i] * s_xh[s][e];
-    } else if (k < OW2) {
-      const int i = k - OB1;
-      for (int s = 0; s < GRAD_BS; ++s) g += s_d1[s][i];
-    } else if (k < OB2) {
-      const int i = (k - OW2) / NH, j = (k - OW2) % NH;
-      for (int s = 0; s < GRAD_BS; ++s) g += s_d2[s][i] * s_h1[s][j];
-    } else if (k < OW3) {
-      const int i = k - OB2;
-      for (int s = 0; s < GRAD_BS; ++s) g += s_d2[s][i];
-    } else if (k < OB3) {
-      const int i = k - OW3;
-      for (int s = 0; s < GRAD_BS; ++s) g += s_d3[s] * s_h2[s][i];
-    } else if (k == OB3) {
-      for (int s = 0; s < GRAD_BS; ++s) g += s_d3[s];
-    } else {
-      for (int s = 0; s < GRAD_BS; ++s) g += s_loss[s];
+#pragma unroll
+  for (int e = 0; e < NIN; ++e) xh[e] = (xh[e] - s_p[OMEAN + e]) * s_p[OISTD + e];
+  if (w == 0) {
+#pragma unroll
+    for (int e = 0; e < NIN; ++e) s_xb[e][lane] = xh[e];
+    s_xb[NIN][lane] = 1.0f;
+  }
+  float z1[U], z2[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = u0 + u;
+    float a = s_p[OB1 + i];
+#pragma unroll
+    for (int e = 0; e < NIN; ++e) a += s_p[OW1 + i * NIN + e] * xh[e];
+    z1[u] = a;
+    s_h1[i][lane] = fmaxf(a, 0.0f);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u) z2[u] = s_p[OB2 + u0 + u];
+#pragma unroll
+  for (int j = 0; j < NH; j += 4) {
+    const float h0 = s_h1[j][lane], h1 = s_h1[j + 1][lane], h2 = s_h1[j + 2][lane], h3 = s_h1[j + 3][lane];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const f32x4 wt = *reinterpret_cast<const f32x4*>(&s_p[OW2 + (u0 + u) * NH + j]);
+      z2[u] = fmaf(wt[3], h3, fmaf(wt[2], h2, fmaf(wt[1], h1, fmaf(wt[0], h0, z2[u]))));
     }
-    out[k] = g;
+  }
+  float part = 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float h = fmaxf(z2[u], 0.0f);
+    s_h2[u0 + u][lane] = h;
+    part += s_p[OW3 + u0 + u] * h;
+  }
+  s_z3[w][lane] = part;
+  __syncthreads();
+  const float z3 = s_p[OB3] + ((s_z3[0][lane] + s_z3[1][lane]) + (s_z3[2][lane] + s_z3[3][lane]));
+  const float res = ok ? softplus(z3) - target : 0.0f;
+  // dL/dz3 = 2 (y - t)/N * softplus'(z3): sigmoid(beta z3), 1 where softplus returns z3 (beta z3 > 20)
+  const float bz = fmaxf(BETA * z3, -60.0f);
+  const float d3 = 2.0f * res * inv_n * (bz > 20.0f ? 1.0f : 1.0f / (1.0f + __expf(-bz)));
+  if (w == 0) s_d3[lane] = d3;
+#pragma unroll
+  for (int u = 0; u < U; ++u) s_d2[u0 + u][lane] = z2[u] > 0.0f ? d3 * s_p[OW3 + u0 + u] : 0.0f;
+  __syncthreads();
+  float d1[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) d1[u] = 0.0f;
+#pragma unroll 8
+  for (int i = 0; i < NH; ++i) {
+    const float d = s_d2[i][lane];
+#pragma unroll
+    for (int u = 0; u < U; u += 4) {
+      const f32x4 wt = *reinterpret_cast<const f32x4*>(&s_p[OW2 + i * NH + u0 + u]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d1[u + e] = fmaf(d, wt[e], d1[u + e]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) s_d1[u0 + u][lane] = z1[u] > 0.0f ? d1[u] : 0.0f;
+  __syncthreads();
+
+  float* out = partials + uint64_t(blockIdx.x) * (NPARAM + 1);
+  const int c = lane & 15, r0 = 4 * (lane >> 4);
+  {  // W2: one quadrant per wave
+    const int i0 = 16 * (w >> 1), j0 = 16 * (w & 1);
+    const f32x4 d = grad_tile(lane, [&](int i, int sm) { return s_d2[i0 + i][sm]; },
+                              [&](int j, int sm) { return s_h1[j0 + j][sm]; });
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[OW2 + (i0 + r0 + r) * NH + j0 + c] = d[r];
+  }
+  const int i0 = 16 * (w & 1);
+  if (w < 2) {  // W1 and b1 (column 7: the ones); then the output weights
+    f32x4 d = grad_tile(lane, [&](int i, int sm) { return s_d1[i0 + i][sm]; },
+                        [&](int j, int sm) { return j < 8 ? s_xb[j][sm] : 0.0f; });
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + r0 + r;
+      if (c < NIN) out[OW1 + i * NIN + c] = d[r];
+      if (c == NIN) out[OB1 + i] = d[r];
+    }
+    d = grad_tile(lane, [&](int i, int sm) { return s_h2[i0 + i][sm]; },
+                  [&](int j, int sm) { return j == 0 ? s_d3[sm] : 0.0f; });
+    if (c == 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[OW3 + i0 + r0 + r] = d[r];
+    }
+  } else {  // b2, b3 and the loss
+    const f32x4 d = grad_tile(lane, [&](int i, int sm) { return s_d2[i0 + i][sm]; },
+                              [&](int j, int) { return j == 0 ? 1.0f : 0.0f; });
+    if (c == 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[OB2 + i0 + r0 + r] = d[r];
+    }
+    const float sum = wave_sum64(w == 2 ? d3 : res * res * inv_n);
+    if (lane == 0) out[w == 2 ? OB3 : NPARAM] = sum;
   }
 }
 
-// One workgroup: sum the per-workgroup partials in block order, clip the
-// global gradient norm (torch.nn.utils.clip_grad_norm_ rule: scale by
-// min(1, clip / (|g| + 1e-6)), ai/train.py:401-405), then one Adam step.
+// One workgroup: sum the per-workgroup partials in a fixed order, clip the global
+// gradient norm (torch.nn.utils.clip_grad_norm_ rule: scale by min(1, clip / (|g| +
+// 1e-6)), ai/train.py:401-405), then one Adam step.  The partials are read four
+// columns to a thread and three interleaved sets of rows at a time, so that a CU has
+// 1011 sixteen-byte loads in flight per row triple (one four-byte column per thread
+// and all rows in turn took 32 us for 64 partials).  loss_sum, when given, receives
+// += loss * weight in double (an epoch's running loss).
 constexpr int ADAM_THREADS = 1024;
+constexpr int COLS4 = (NPARAM + 1 + 3) / 4;           // 337
+constexpr int ROW_SETS = ADAM_THREADS / COLS4;        // 3
 static_assert(2 * ADAM_THREADS > NPARAM, "two entries per thread cover the gradient and the loss");
+static_assert(ROW_SETS == 3, "sums of three row sets");
+// rows are 4-byte aligned (an odd number of float pairs apart)
+struct __attribute__((packed, aligned(4))) Row4 {
+  float v[4];
+};
 
 __global__ __launch_bounds__(ADAM_THREADS) void k_mlp_adam(float* __restrict__ p, const float* __restrict__ partials,
                                                            int nblk, float* __restrict__ m, float* __restrict__ v,
                                                            float lr, float b1, float b2, float eps, float bc1,
                                                            float bc2, float clip, float* __restrict__ loss_out,
-                                                           float* __restrict__ grad_out) {
-  __shared__ float s_red[ADAM_THREADS];
+                                                           float* __restrict__ grad_out,
+                                                           double* __restrict__ loss_sum, double weight) {
+  __shared__ float s_g[ROW_SETS][4 * COLS4];
+  __shared__ float s_red[ADAM_THREADS / 64];
   const int tid = threadIdx.x;
+  const bool update = lr != 0.0f;
+  float pk[2] = {}, mk[2] = {}, vk[2] = {};
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int k = tid + r * ADAM_THREADS;
+    if (update && k < NPARAM) {
+      pk[r] = p[k];
+      mk[r] = m[k];
+      vk[r] = v[k];
+    }
+  }
+  const int set = tid / COLS4, col = 4 * (tid % COLS4);
+  if (set < ROW_SETS) {
+    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const float* src = partials + col;
+    if (col + 4 <= NPARAM + 1) {
+#pragma unroll 8
+      for (int b = set; b < nblk; b += ROW_SETS) {
+        const Row4 q = *reinterpret_cast<const Row4*>(src + uint64_t(b) * (NPARAM + 1));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] += q.v[e];
+      }
+    } else {  // the last columns of a row
+      for (int b = set; b < nblk; b += ROW_SETS)
+        for (int e = 0; col + e <= NPARAM; ++e) a[e] += src[uint64_t(b) * (NPARAM + 1) + e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s_g[set][col + e] = a[e];
+  }
+  __syncthreads();
   float g[2];
   float sq = 0.0f;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     const int k = tid + r * ADAM_THREADS;
-    float a = 0.0f;
-    if (k <= NPARAM)
-      for (int b = 0; b < nblk; ++b) a += partials[uint64_t(b) * (NPARAM + 1) + k];
-    g[r] = a;
-    if (k < NPARAM) sq += a * a;
+    g[r] = k <= NPARAM ? (s_g[0][k] + s_g[1][k]) + s_g[2][k] : 0.0f;
+    if (k < NPARAM) sq += g[r] * g[r];
   }
-  s_red[tid] = sq;
+  sq = wave_sum64(sq);
+  if ((tid & 63) == 0) s_red[tid >> 6] = sq;
   __syncthreads();
-  for (int off = ADAM_THREADS / 2; off > 0; off >>= 1) {
-    if (tid < off) s_red[tid] += s_red[tid + off];
-    __syncthreads();
-  }
-  const float norm = sqrtf(s_red[0]);
+  float total = 0.0f;
+#pragma unroll
+  for (int i = 0; i < ADAM_THREADS / 64; ++i) total += s_red[i];
+  const float norm = sqrtf(total);
   const float scale = clip > 0.0f ? fminf(1.0f, clip / (norm + 1e-6f)) : 1.0f;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     const int k = tid + r * ADAM_THREADS;
-    if (k == NPARAM && loss_out) *loss_out = g[r];
+    if (k == NPARAM) {
+      if (loss_out) *loss_out = g[r];
+      if (loss_sum) *loss_sum += double(g[r]) * weight;
+    }
     if (k >= NPARAM) continue;
     if (grad_out) grad_out[k] = g[r];
-    if (lr == 0.0f) continue;
+    if (!update) continue;
     const float gk = g[r] * scale;
-    const float mk = b1 * m[k] + (1.0f - b1) * gk;
-    const float vk = b2 * v[k] + (1.0f - b2) * gk * gk;
-    m[k] = mk;
-    v[k] = vk;
-    p[k] -= lr * (mk / bc1) / (sqrtf(vk / bc2) + eps);
+    mk[r] = b1 * mk[r] + (1.0f - b1) * gk;
+    vk[r] = b2 * vk[r] + (1.0f - b2) * gk * gk;
+    m[k] = mk[r];
+    v[k] = vk[r];
+    p[k] = pk[r] - lr * (mk[r] / bc1) / (sqrtf(vk[r] / bc2) + eps);
   }
 }
 
@@ -417,8 +546,8 @@ int tlbm_mlp_grad(const float* params, const float* x, const float* t, int64_t n
   if (!params || !x || !t || !partials) return cfail(TLBM_ERR_INVALID, "null pointer");
   const uint64_t nb = (uint64_t(n) + GRAD_BS - 1) / GRAD_BS;
   if (nb >= (uint64_t(1) << 31)) return cfail(TLBM_ERR_SHAPE, "batch too large");
-  hipLaunchKernelGGL(k_mlp_grad, dim3(uint32_t(nb)), dim3(256), 0, (hipStream_t)stream, params, x, t, uint64_t(n),
-                     1.0f / float(n), partials);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(uint32_t(nb)), dim3(256), 0, (hipStream_t)stream, params, x, t,
+                     (const int64_t*)nullptr, uint64_t(n), 1.0f / float(n), partials);
   return claunch("k_mlp_grad");
 }
 
@@ -430,7 +559,7 @@ int tlbm_mlp_adam(float* params, const float* partials, int nblocks, float* m, f
   const float bc1 = 1.0f - powf(beta1, float(step));
   const float bc2 = 1.0f - powf(beta2, float(step));
   hipLaunchKernelGGL(k_mlp_adam, dim3(1), dim3(ADAM_THREADS), 0, (hipStream_t)stream, params, partials, nblocks, m,
-                     v, lr, beta1, beta2, eps, bc1, bc2, clip_norm, loss_out, grad_out);
+                     v, lr, beta1, beta2, eps, bc1, bc2, clip_norm, loss_out, grad_out, (double*)nullptr, 0.0);
   return claunch("k_mlp_adam");
 }
 
@@ -451,14 +580,14 @@ int tlbm_mlp_train_step_noalloc(float* params, const float* x, const float* t, i
   if (rc != TLBM_OK) return rc;
   const int nb = int((n + GRAD_BS - 1) / GRAD_BS);
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_mlp_grad, dim3(uint32_t(nb)), dim3(256), 0, s, params, x, t, uint64_t(n), 1.0f / float(n),
-                     partials);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(uint32_t(nb)), dim3(256), 0, s, params, x, t, (const int64_t*)nullptr,
+                     uint64_t(n), 1.0f / float(n), partials);
   const int rg = claunch("k_mlp_grad");
   if (rg != TLBM_OK) return rg;
   const float bc1 = 1.0f - powf(beta1, float(step));
   const float bc2 = 1.0f - powf(beta2, float(step));
   hipLaunchKernelGGL(k_mlp_adam, dim3(1), dim3(ADAM_THREADS), 0, s, params, partials, nb, m, v, lr, beta1, beta2,
-                     eps, bc1, bc2, clip_norm, loss_out, grad_out);
+                     eps, bc1, bc2, clip_norm, loss_out, grad_out, (double*)nullptr, 0.0);
   return claunch("k_mlp_adam");
 }
 
