@@ -299,6 +299,19 @@ int tlbm_mlp_train_step_noalloc(float* params, const float* x, const float* t, i
                                 tlbm_stream_t stream);
 
 /*
+ * One epoch of minibatch training (the inner loop of train_eddy_viscosity_model, ai/train.py:382-435):
+ * for every `batch` consecutive entries of order[n] (row numbers of x and t; the last minibatch may be
+ * smaller) the gradient of that minibatch, clipping and one Adam step, numbered from `step` on.  The
+ * same rule as tlbm_mlp_grad + tlbm_mlp_adam on the gathered rows (sums in another fixed order), three
+ * launches per minibatch and no copy of its rows.  workspace holds (ceil(batch / batch_block) + 1) *
+ * (nparam + 1) floats and may be reused by the caller's next call on the same stream.
+ * loss_sum[0] receives += (minibatch MSE) * (its size), in double.
+ */
+int tlbm_mlp_train_epoch(float* params, const float* x, const float* t, const int64_t* order, int64_t n,
+                         int64_t batch, float* workspace, float* m, float* v, int step, float lr, float beta1,
+                         float beta2, float eps, float clip_norm, double* loss_sum, tlbm_stream_t stream);
+
+/*
  * The reference's 2-D learned closure (EddyViscosityMLP, ai/model.py:19-92): an MLP in -> H -> ... -> H -> 1
  * with hidden activation tanh / relu / gelu (exact erf form) and a Softplus(beta = 10) output.  Parameters are
  * one fp32 vector in nn.Sequential order -- per hidden layer W [H][in] then b [H], then the output w [H] and

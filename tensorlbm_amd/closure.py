@@ -215,6 +215,24 @@ class _Adam:
         self.model.mark_updated()
         return self.loss
 
+    def epoch(self, x: torch.Tensor, t: torch.Tensor, order: torch.Tensor, batch: int) -> torch.Tensor:
+        """Steps over ``order`` in minibatches of ``batch`` rows; Σ MSE · size as a float64 device scalar.
+
+        The kernels take their rows of ``x`` and ``t`` through ``order``, so a minibatch is three launches
+        and no copy."""
+        n = int(order.shape[0])
+        rows = (min(int(batch), n) + self.bb - 1) // self.bb
+        work = torch.empty((rows + 1, self.model.nparam + 1), dtype=torch.float32, device=self.model.device)
+        total = torch.zeros((), dtype=torch.float64, device=self.model.device)
+        nat.check(nat.lib().tlbm_mlp_train_epoch(self.model.params.data_ptr(), x.data_ptr(), t.data_ptr(),
+                                                 order.data_ptr(), n, min(int(batch), n), work.data_ptr(),
+                                                 self.m.data_ptr(), self.v.data_ptr(), self.t + 1, self.lr, self.b1,
+                                                 self.b2, self.eps, self.clip, total.data_ptr(), nat.stream_of(x)),
+                  "tlbm_mlp_train_epoch")
+        self.t += (n + int(batch) - 1) // int(batch)
+        self.model.mark_updated()
+        return total
+
 
 @dataclass
 class TrainConfig3D:
@@ -270,12 +288,7 @@ def train_eddy_viscosity_model_3d(features: torch.Tensor, targets: torch.Tensor,
     t0 = time.perf_counter()
     for epoch in range(int(cfg.epochs)):
         order = torch.randperm(n_tr, generator=gen).to(device)
-        ep_loss = torch.zeros((), dtype=torch.float64, device=device)
-        for s in range(0, n_tr, bs):
-            idx = order[s:s + bs]
-            xb = x_tr.index_select(0, idx).contiguous()
-            yb = y_tr.index_select(0, idx).contiguous()
-            ep_loss += opt.step(xb, yb)[0].double() * xb.shape[0]
+        ep_loss = opt.epoch(x_tr, y_tr, order, bs)
         pred = model(x_val).reshape(-1)
         val_mse = float(torch.mean((pred - y_val) ** 2))
         met = {"epoch": epoch, "train_mse": float(ep_loss) / n_tr, "val_mse": val_mse,

@@ -55,3 +55,39 @@ def test_predict_matches_float64(n):
     got = model(x.to("cuda:0")).reshape(-1).double().cpu()
     # softplus at slope <= 1 of a sum of 32 products of O(1): a few ulp of fp32 on z
     assert float((got - want).abs().max()) <= 4e-6
+
+
+@pytest.mark.parametrize("n,batch", [(1, 8), (64, 64), (130, 64), (1000, 96), (1000, 1000), (333, 1)])
+def test_epoch_matches_single_steps(n, batch):
+    """The epoch's gathered rows, last short minibatch, step numbers and loss sum, against one step at a time.
+
+    Both sum the same partials, in another order: parameters differ by rounding (Adam's step is at most lr
+    per parameter, so a relative difference of 1e-4 in a gradient near zero moves one by 1e-4 lr)."""
+    a, x, t = _case(n, 3 * n + batch)
+    b = cl.clone_model(a)
+    x, t = x.to("cuda:0"), t.to("cuda:0")
+    order = torch.randperm(n, generator=torch.Generator().manual_seed(n)).to("cuda:0")
+    oa, ob = (cl._Adam(m, 1e-3, max_batch=batch) for m in (a, b))
+    want, steps = 0.0, 0
+    for s in range(0, n, batch):
+        idx = order[s:s + batch]
+        want += float(oa.step(x[idx].contiguous(), t[idx].contiguous())[0].double()) * idx.shape[0]
+        steps += 1
+    got = float(ob.epoch(x, t, order, batch))
+    assert oa.t == ob.t == steps
+    assert abs(got - want) <= 1e-5 * abs(want)
+    assert float((a.params - b.params).abs().max()) <= 1e-3 * 1e-3 * steps
+    assert float((oa.m - ob.m).abs().max()) <= 1e-4 * float(oa.m.abs().max())
+
+
+def test_epoch_refuses_bad_arguments():
+    from tensorlbm_amd import _native as nat
+
+    lib = nat.lib()
+    ok = (4096,) * 4
+    tail = (4096, 4096, 4096)
+    rates = (1e-3, 0.9, 0.999, 1e-8, 1.0)
+    assert lib.tlbm_mlp_train_epoch(*ok, 0, 8, *tail, 1, *rates, 4096, None) == nat.ERR_SHAPE
+    assert lib.tlbm_mlp_train_epoch(*ok, 8, 0, *tail, 1, *rates, 4096, None) == nat.ERR_SHAPE
+    assert lib.tlbm_mlp_train_epoch(*ok, 8, 8, *tail, 0, *rates, 4096, None) == nat.ERR_INVALID
+    assert lib.tlbm_mlp_train_epoch(*ok, 8, 8, *tail, 1, *rates, None, None) == nat.ERR_INVALID
