@@ -236,6 +236,29 @@ int tlbm_boundary_eager(int dtype, const void* f_in, void* f_out, int nz, int ny
                         const tlbm_boundary* bc, const int8_t* mask_a, const int8_t* mask_b,
                         tlbm_stream_t stream);
 
+/*
+ * The six far-field faces of the obstacle loop, in place (apply_far_field_bc_6face,
+ * triton_fused_obstacle.py:2386-2471): f (q, nz, ny, nx), q >= 19, element strides (q, z, y) and unit x
+ * stride, no two elements in one place; storage F32, F64, F16 or BF16 (absolute populations).  x = 0
+ * takes the face value, x = nx-1 a copy of x = nx-2, then y = 0, y = ny-1 and, when nz > 4, z = 0 and
+ * z = nz-1 take the face value.  The face values are feq (device, q values of the storage type) or,
+ * with feq NULL, f_eq(1, u) in double rounded to F32 / F64 (q = 19; u: 3 host doubles).
+ */
+int tlbm_far_field_faces(int store, int q, void* f, const int64_t* strides, int nz, int ny, int nx, const double* u,
+                         const void* feq, tlbm_stream_t stream);
+
+/* fx[0] += acc[0], fy[0] += acc[1], fz[0] += acc[2] (device; dtype F32 or F64), the step's FP64 force
+ * sample into a caller's buffers (triton_fused_obstacle.py:1494-1512) */
+int tlbm_force_add(int dtype, const double* acc, void* fx, void* fy, void* fz, tlbm_stream_t stream);
+
+/* f <- f * (target / sum f), unchanged where |sum f| < 1e-30 (apply_mass_correction,
+ * triton_fused_obstacle.py:2513-2527), the sum in FP64 and in a fixed order; storage F32, F64, F16 or
+ * BF16.  workspace: TLBM_MASS_WORKSPACE device doubles.  TLBM_ERR_UNSUPPORTED where the (y, x) planes
+ * are not contiguous (use tlbm_moment_sums and tlbm_scale). */
+#define TLBM_MASS_WORKSPACE 1024
+int tlbm_mass_correct(int lattice, int store, void* f, const int64_t* strides, int nz, int ny, int nx, double target,
+                      double* workspace, tlbm_stream_t stream);
+
 /* sphere_mask (boundaries3d.py:29-49): out[z][y][x] = 1 where (x-cx)^2 + (y-cy)^2 + (z-cz)^2 <=
  * radius^2, else 0, evaluated in float32 as the reference does (centre rounded to float32, squares
  * and sums rounded in turn, radius^2 formed in double and rounded to float32); out holds nz*ny*nx

@@ -60,6 +60,7 @@ class Cavity(ctypes.Structure):
 
 CAVITIES_MAX = 128
 MLP_NOALLOC_MAX_SAMPLES = 32768  # TLBM_MLP_NOALLOC_MAX_SAMPLES
+MASS_WORKSPACE = 1024  # TLBM_MASS_WORKSPACE
 
 
 class Boundary(ctypes.Structure):
@@ -113,6 +114,9 @@ _SIGNATURES = {
     "tlbm_obstacle_force": ([_I, _I, _VP, _VP, _I, _I, _I, _VP, _VP, _VP], _I),
     "tlbm_scale": ([_I, _I, _VP, _VP, _I, _I, _I, _VP, _VP], _I),
     "tlbm_boundary_eager": ([_I, _VP, _VP, _I, _I, _I, ctypes.POINTER(Boundary), _VP, _VP, _VP], _I),
+    "tlbm_far_field_faces": ([_I, _I, _VP, _VP, _I, _I, _I, ctypes.POINTER(ctypes.c_double), _VP, _VP], _I),
+    "tlbm_force_add": ([_I, _VP, _VP, _VP, _VP, _VP], _I),
+    "tlbm_mass_correct": ([_I, _I, _VP, _VP, _I, _I, _I, ctypes.c_double, _VP, _VP], _I),
     "tlbm_sphere_mask": ([_I, _I, _I, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double, _VP,
                           _VP], _I),
     "tlbm_gradient_closure_tau": ([_I, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, ctypes.c_double, ctypes.c_double,

@@ -1395,6 +1395,147 @@ __global__ __launch_bounds__(256) void k_scale(void* fv, Layout lay, const doubl
   }
 }
 
+// ---------------------------------------------------------------------------
+// companions of the obstacle step
+// ---------------------------------------------------------------------------
+
+// The six far-field faces written in place (triton_fused_obstacle.py:2386-2471): the
+// population's face value on x = 0, a copy of x = nx-2 on x = nx-1, then the face
+// value on the y planes and, when `zfaces`, on the z planes; later faces win on shared
+// edges, so every cell is written once with the value the last of them leaves.  The
+// outlet reads x = nx-2, which no face of its row writes (nx = 2: the inlet's value).
+// One launch instead of a plane copy per face and the small operators that built the
+// face value: 96 x 96 x 193 fp32, about 25 launches -> one of 15 us.  Lanes enumerate a
+// population's face cells: first the (z, y) pairs of the x faces, whose two cells lie
+// next to each other in memory (x = nx-1 of a row, x = 0 of the next), then the rows
+// of the y faces and the z planes, contiguous.  blockIdx.y: population.
+struct FaceValues {
+  double v[19];
+};
+template <typename T>
+__global__ __launch_bounds__(256) void k_faces(T* f, int64_t sq, int64_t sz, int64_t sy, int nz, int ny, int nx,
+                                               int zfaces, const T* feq, const FaceValues fv) {
+  const int q = int(blockIdx.y);
+  const T face = feq != nullptr ? feq[q] : T(fv.v[q < 19 ? q : 0]);
+  T* fq = f + int64_t(q) * sq;
+  const int z0 = zfaces ? 1 : 0, zn = zfaces ? nz - 2 : nz;  // z planes left to the x and y faces
+  const int yn = ny > 2 ? ny - 2 : 0, yf = ny >= 2 ? 2 : 1;  // y rows left to the x faces; y faces
+  const uint64_t na = uint64_t(zn) * uint64_t(yn), nb = uint64_t(zn) * uint64_t(yf) * uint64_t(nx);
+  const uint64_t nc = zfaces ? uint64_t(2) * uint64_t(ny) * uint64_t(nx) : 0;
+  for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < na + nb + nc;
+       i += uint64_t(gridDim.x) * blockDim.x) {
+    if (i < na) {
+      T* row = fq + int64_t(z0 + int(uint32_t(i) / uint32_t(yn))) * sz + int64_t(1 + int(uint32_t(i) % uint32_t(yn))) * sy;
+      const T out = nx > 2 ? row[nx - 2] : face;
+      row[0] = face;
+      if (nx >= 2) row[nx - 1] = out;
+    } else if (i < na + nb) {
+      const uint32_t k = uint32_t(i - na), r = k / uint32_t(nx), x = k - r * uint32_t(nx);
+      const int z = z0 + int(r / uint32_t(yf)), y = int(r % uint32_t(yf)) * (ny - 1);
+      fq[int64_t(z) * sz + int64_t(y) * sy + x] = face;
+    } else {
+      const uint32_t k = uint32_t(i - na - nb), r = k / uint32_t(nx), x = k - r * uint32_t(nx);
+      const int z = int(r / uint32_t(ny)) * (nz - 1), y = int(r % uint32_t(ny));
+      fq[int64_t(z) * sz + int64_t(y) * sy + x] = face;
+    }
+  }
+}
+
+// b[i] += acc[i], i = 0..2, in turn (the buffers may be one and the same)
+template <typename T>
+__global__ void k_force_add(const double* acc, T* bx, T* by, T* bz) {
+  *bx += T(acc[0]);
+  *by += T(acc[1]);
+  *bz += T(acc[2]);
+}
+
+// Sum and rescale of a whole lattice as `planes` runs of `len` contiguous values, run p
+// at (p / inner_n) * outer + (p % inner_n) * inner.  A workgroup takes pieces of
+// MASS_PIECE values, four neighbouring ones to a lane and eight loads in flight; runs
+// start at any element, which global memory operations allow.  The per-cell forms (k_moment_sums: four
+// FP64 sums and two 64-bit divisions per cell; k_scale) took 58 and 44 us on
+// 96 x 96 x 193 fp32; these take 24 and 42 us.  The sum leaves one FP64 partial per
+// workgroup, added up in a fixed order by every workgroup of the scaling, so there is
+// no atomic, nothing to clear and the result does not vary from run to run.
+constexpr int MASS_PIECE = 256 * 4 * 8;
+constexpr int MASS_BLOCKS = 1024;
+struct Runs {
+  int64_t outer, inner, len;
+  uint32_t planes, inner_n, pieces;  // pieces per run
+};
+// four values from an address aligned like one of them (at least two bytes)
+template <typename T>
+struct Vec4 {
+  typedef T type __attribute__((ext_vector_type(4), aligned(sizeof(T) < 4 ? sizeof(T) : 4)));
+};
+
+// fn4(values, address) on groups of four, fn1(value, address) on the last values of a run
+template <int S, class F4, class F1>
+__device__ __forceinline__ void for_pieces(typename Store<S>::T* f, const Runs& r, const F4& fn4, const F1& fn1) {
+  using T = typename Store<S>::T;
+  using V = typename Vec4<T>::type;
+  const uint64_t units = uint64_t(r.planes) * r.pieces;
+  for (uint64_t u = blockIdx.x; u < units; u += gridDim.x) {
+    const uint32_t p = uint32_t(u / r.pieces), k = uint32_t(u % r.pieces);
+    const int64_t at = int64_t(k) * MASS_PIECE;
+    T* base = f + int64_t(p / r.inner_n) * r.outer + int64_t(p % r.inner_n) * r.inner + at;
+    const int64_t left = r.len - at;
+    const uint32_t lane = threadIdx.x * 4;
+    if (left >= MASS_PIECE) {
+      V v[8];
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) v[j] = *(global_ptr<const V>)(base + (lane + j * 1024));
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) fn4(v[j], (global_ptr<V>)(base + (lane + j * 1024)));
+    } else {
+      for (int64_t i = threadIdx.x; i < left; i += 256) fn1(base[i], (global_ptr<T>)(base + i));
+    }
+  }
+}
+
+template <class L, int S>
+__global__ __launch_bounds__(256) void k_mass_sum(const void* fv, Runs r, double* partial) {
+  using T = typename Store<S>::T;
+  using V = typename Vec4<T>::type;
+  double a[4] = {0.0, 0.0, 0.0, 0.0};
+  for_pieces<S>(
+      static_cast<T*>(const_cast<void*>(fv)), r,
+      [&](const V& v, global_ptr<V>) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] += double(Store<S>::template get<L>(v[e], 0));
+      },
+      [&](T v, global_ptr<T>) { a[0] += double(Store<S>::template get<L>(v, 0)); });
+  const double s = wave_sum((a[0] + a[1]) + (a[2] + a[3]));
+  __shared__ double part[4];
+  if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) partial[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+}
+
+// f *= target / sum(partial), or 1 where the sum vanishes (triton_fused_obstacle.py:2513-2527)
+template <class L, int S>
+__global__ __launch_bounds__(256) void k_mass_scale(void* fv, Runs r, const double* partial, int npartial,
+                                                    double target) {
+  using T = typename Store<S>::T;
+  double s = 0.0;
+  for (int i = threadIdx.x; i < npartial; i += 256) s += partial[i];
+  s = wave_sum(s);
+  __shared__ double part[4];
+  if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = s;
+  __syncthreads();
+  s = (part[0] + part[1]) + (part[2] + part[3]);
+  const typename Store<S>::C scale = typename Store<S>::C(fabs(s) < 1e-30 ? 1.0 : target / s);
+  using V = typename Vec4<T>::type;
+  for_pieces<S>(
+      static_cast<T*>(fv), r,
+      [&](V v, global_ptr<V> at) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = Store<S>::template put<L>(Store<S>::template get<L>(v[e], 0) * scale, 0);
+        *at = v;
+      },
+      [&](T v, global_ptr<T> at) { *at = Store<S>::template put<L>(Store<S>::template get<L>(v, 0) * scale, 0); });
+}
+
 }  // namespace tlbm
 
 // ===========================================================================
@@ -2347,6 +2488,101 @@ int tlbm_scale(int lattice, int store, void* f, const int64_t* strides, int nz, 
       hipLaunchKernelGGL((k_scale<L, S>), dim3(blocks_for(n)), dim3(256), 0, s, f, lay, scale);
       return check_launch("k_scale");
     });
+  });
+}
+
+int tlbm_far_field_faces(int store, int q, void* f, const int64_t* strides, int nz, int ny, int nx, const double* u,
+                         const void* feq, tlbm_stream_t stream) {
+  g_err[0] = 0;
+  if (q < 19 || q > 65535) return fail(TLBM_ERR_SHAPE, "need 19..65535 populations (got %d)", q);
+  if (store < TLBM_STORE_F32 || store > TLBM_STORE_BF16) return fail(TLBM_ERR_DTYPE, "unknown storage %d", store);
+  int rc = check_dims(TLBM_D3Q19, nz, ny, nx);
+  if (rc) return rc;
+  if (!f || !strides || (!u && !feq)) return fail(TLBM_ERR_INVALID, "null pointer");
+  if (!feq && (q != 19 || (store != TLBM_STORE_F32 && store != TLBM_STORE_F64)))
+    return fail(TLBM_ERR_INVALID, "face values from u are for 19 float32 or float64 populations; pass feq");
+  FaceValues fv = {};
+  if (!feq) {  // f_eq(1, u) in double
+    const double uu = 1.5 * (u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+    for (int k = 0; k < 19; ++k) {
+      const double cu = D3Q19::cx[k] * u[0] + D3Q19::cy[k] * u[1] + D3Q19::cz[k] * u[2];
+      fv.v[k] = D3Q19::w[k] * (1.0 + 3.0 * cu + 4.5 * cu * cu - uu);
+    }
+  }
+  const int zfaces = nz > 4 ? 1 : 0;
+  const uint64_t cells = uint64_t(nz) * ny + 2 * (uint64_t(nz) * nx) + (zfaces ? 2 * uint64_t(ny) * nx : 0);
+  const uint64_t nb = (cells + 255) / 256;
+  const dim3 grid(uint32_t(nb < 65536 ? nb : 65536), uint32_t(q));
+  hipStream_t s = (hipStream_t)stream;
+  const auto go = [&](auto* p) -> int {
+    using T = std::remove_pointer_t<decltype(p)>;
+    hipLaunchKernelGGL(k_faces<T>, grid, dim3(256), 0, s, p, strides[0], strides[1], strides[2], nz, ny, nx, zfaces,
+                       static_cast<const T*>(feq), fv);
+    return check_launch("k_faces");
+  };
+  switch (store) {
+    case TLBM_STORE_F32: return go(static_cast<float*>(f));
+    case TLBM_STORE_F64: return go(static_cast<double*>(f));
+    case TLBM_STORE_F16: return go(static_cast<_Float16*>(f));
+    default: return go(static_cast<uint16_t*>(f));
+  }
+}
+
+int tlbm_force_add(int dtype, const double* acc, void* fx, void* fy, void* fz, tlbm_stream_t stream) {
+  g_err[0] = 0;
+  if (!acc || !fx || !fy || !fz) return fail(TLBM_ERR_INVALID, "null pointer");
+  hipStream_t s = (hipStream_t)stream;
+  if (dtype == TLBM_STORE_F32) {
+    hipLaunchKernelGGL(k_force_add<float>, dim3(1), dim3(1), 0, s, acc, (float*)fx, (float*)fy, (float*)fz);
+  } else if (dtype == TLBM_STORE_F64) {
+    hipLaunchKernelGGL(k_force_add<double>, dim3(1), dim3(1), 0, s, acc, (double*)fx, (double*)fy, (double*)fz);
+  } else {
+    return fail(TLBM_ERR_DTYPE, "force buffers are float32 or float64");
+  }
+  return check_launch("k_force_add");
+}
+
+int tlbm_mass_correct(int lattice, int store, void* f, const int64_t* strides, int nz, int ny, int nx, double target,
+                      double* workspace, tlbm_stream_t stream) {
+  g_err[0] = 0;
+  int rc = check_dims(lattice, nz, ny, nx);
+  if (rc) return rc;
+  if (store < TLBM_STORE_F32 || store > TLBM_STORE_BF16)
+    return fail(TLBM_ERR_DTYPE, "mass correction takes absolute populations");
+  if (!f || !workspace) return fail(TLBM_ERR_INVALID, "null pointer");
+  int64_t st[3];
+  rc = resolve_strides(strides, lattice, nz, ny, nx, store_size(store), st, "f");
+  if (rc) return rc;
+  // contiguous runs: the whole lattice, its (z, q) planes, or single rows
+  const int64_t plane = int64_t(ny) * nx;
+  Runs r;
+  if (st[2] == nx && (nz == 1 || st[1] == plane) && st[0] == plane * nz) {
+    r = Runs{0, 0, plane * nz * lattice, 1, 1, 0};
+  } else if (st[2] == nx || ny == 1) {
+    r = Runs{st[1], st[0], plane, uint32_t(nz) * uint32_t(lattice), uint32_t(lattice), 0};
+  } else {
+    return fail(TLBM_ERR_UNSUPPORTED, "mass correction needs contiguous (y, x) planes");
+  }
+  const int64_t pieces = (r.len + MASS_PIECE - 1) / MASS_PIECE;
+  r.pieces = uint32_t(pieces);
+  const uint64_t units = uint64_t(pieces) * r.planes;
+  const uint32_t nsum = uint32_t(units < MASS_BLOCKS ? units : MASS_BLOCKS);
+  const uint32_t nscale = uint32_t(units < 4 * MASS_BLOCKS ? units : 4 * MASS_BLOCKS);
+  hipStream_t s = (hipStream_t)stream;
+  return by_lattice(lattice, [&](auto lat) -> int {
+    using L = decltype(lat);
+    const auto go = [&](auto sk) -> int {
+      constexpr int S = decltype(sk)::value;
+      hipLaunchKernelGGL((k_mass_sum<L, S>), dim3(nsum), dim3(256), 0, s, f, r, workspace);
+      hipLaunchKernelGGL((k_mass_scale<L, S>), dim3(nscale), dim3(256), 0, s, f, r, workspace, int(nsum), target);
+      return check_launch("k_mass_scale");
+    };
+    switch (store) {
+      case ST_F32: return go(std::integral_constant<int, ST_F32>{});
+      case ST_F64: return go(std::integral_constant<int, ST_F64>{});
+      case ST_F16: return go(std::integral_constant<int, ST_F16>{});
+      default: return go(std::integral_constant<int, ST_BF16>{});
+    }
   });
 }
 

@@ -16,6 +16,7 @@ Drop-in for the reference's fused GPU path:
 
 from __future__ import annotations
 
+import ctypes
 import time
 from typing import Sequence
 
@@ -216,9 +217,32 @@ def fused_obstacle_step(
         acc = torch.zeros(3, dtype=torch.float64, device=f.device)
     _launch_step(f, out, coll, solid=solid, force=acc, what="fused_obstacle_step")
     if force is None and acc is not None:
-        for i, b in enumerate(bufs):
-            b.add_(acc[i].to(b.dtype))
+        dt = fx_buf.dtype
+        if dt in (torch.float32, torch.float64) and all(
+                b.numel() == 1 and b.dtype == dt and b.device == f.device and _plain(b) for b in bufs):
+            nat.check(nat.lib().tlbm_force_add(nat.store_code(dt), acc.data_ptr(), *(b.data_ptr() for b in bufs),
+                                               nat.stream_of(f)), "fused_obstacle_step")
+        else:
+            for i, b in enumerate(bufs):
+                b.add_(acc[i].to(b.dtype))
     return out
+
+
+def _plain(t: torch.Tensor) -> bool:
+    """A tensor that a kernel may write in place without torch seeing it: no subclass, no autograd."""
+    return type(t) is torch.Tensor and not t.requires_grad
+
+
+def _distinct(f: torch.Tensor) -> bool:
+    """No two elements of ``f`` share memory and x is its fastest axis (stride 1)."""
+    if f.stride(-1) != 1:
+        return False
+    span = 1
+    for n, st in sorted(((n, st) for n, st in zip(f.shape, f.stride()) if n > 1), key=lambda v: v[1]):
+        if st < span:
+            return False
+        span = st * n
+    return f.numel() > 0
 
 
 def apply_far_field_bc_6face(f: torch.Tensor, u_in: float, *, uy: float = 0.0, uz: float = 0.0,
@@ -230,14 +254,20 @@ def apply_far_field_bc_6face(f: torch.Tensor, u_in: float, *, uy: float = 0.0, u
 
     ``f`` holds absolute populations, shape ``(Q, nz, ny, nx)`` with Q ≥ 19 (slots past 19 are set to 0,
     as the reference pads its 32-slot buffers).  ``feq_vec`` (shape ``(19,)`` or ``(Q,)``) skips the
-    equilibrium; otherwise it comes from the library's equilibrium kernel on one cell.  These are
-    O(Q·area) plane writes on the device, as in the reference; ``FusedSolver3D(boundary="far_field")``
-    applies the same faces inside the step instead.
+    equilibrium.  One launch writes every face (``tlbm_far_field_faces``; a plane copy each where ``f`` is
+    no plain dense floating-point tensor); ``FusedSolver3D(boundary="far_field")`` applies the same faces
+    inside the step instead.
     """
     if f.dim() != 4 or f.shape[0] < 19:
         raise ValueError(f"f must be (Q >= 19, nz, ny, nx), got shape {tuple(f.shape)}")
     nat.require_gpu(f, "apply_far_field_bc_6face")
     q, nz, ny, nx = (int(v) for v in f.shape)
+    launch = f.dtype in (torch.float32, torch.float64, torch.float16, torch.bfloat16) and _plain(f) and _distinct(f)
+    if launch and feq_vec is None and q == 19 and f.dtype in (torch.float32, torch.float64):
+        u = (ctypes.c_double * 3)(float(u_in), float(uy), float(uz))
+        nat.check(nat.lib().tlbm_far_field_faces(nat.store_code(f.dtype), q, f.data_ptr(), nat.strides_of(f), nz, ny,
+                                                 nx, u, None, nat.stream_of(f)), "apply_far_field_bc_6face")
+        return
     if feq_vec is None:
         from .ops import equilibrium3d
 
@@ -256,6 +286,12 @@ def apply_far_field_bc_6face(f: torch.Tensor, u_in: float, *, uy: float = 0.0, u
         feq_vec = feq_pad_buf
     elif feq_vec.shape[0] > q:
         feq_vec = feq_vec[:q]
+    if launch and _plain(feq_vec):
+        feq_vec = feq_vec.contiguous()
+        nat.check(nat.lib().tlbm_far_field_faces(nat.store_code(f.dtype), q, f.data_ptr(), nat.strides_of(f), nz, ny,
+                                                 nx, None, feq_vec.data_ptr(), nat.stream_of(f)),
+                  "apply_far_field_bc_6face")
+        return
     face = feq_vec[:, None, None]
     f[:, :, :, 0] = face
     if nx >= 2:
@@ -276,6 +312,13 @@ def apply_mass_correction(f: torch.Tensor, target_mass: float) -> torch.Tensor:
     if f.dim() != 4 or q not in (19, 27):
         raise ValueError(f"f must be (19 or 27, nz, ny, nx), got shape {tuple(f.shape)}")
     nat.require_gpu(f, "apply_mass_correction")
+    if f.numel() > 0 and f.stride(2) == f.shape[3] and _distinct(f):
+        work = torch.empty(nat.MASS_WORKSPACE, dtype=torch.float64, device=f.device)
+        nz, ny, nx = (int(v) for v in f.shape[1:])
+        nat.check(nat.lib().tlbm_mass_correct(q, nat.store_code(f.dtype), f.data_ptr(), nat.strides_of(f), nz, ny, nx,
+                                              float(target_mass), work.data_ptr(), nat.stream_of(f)),
+                  "apply_mass_correction")
+        return f
     from .ops import moment_sums
 
     cur = moment_sums(f)[0:1]
