@@ -862,6 +862,131 @@ __device__ __forceinline__ void geier27(C (&f)[27], C rho_eq, const Macro<C>& mc
   populations<L>(m, f);
 }
 
+// geier27 for omega_b = omega_odd = omega_even = 1 (the reference's defaults): every
+// cumulant but the trace-free second-order ones becomes the equilibrium's, so only the
+// ten moments up to second order are taken from f (66 additions against 81 and three
+// shifts), no cumulant above second order is formed from f, and the central moments
+// follow from the second-order cumulants and the closed forms of eq_cumulants27, all
+// per unit mass (k = kappa / rho, s_ab = C_ab / rho):
+//   k_210 = -ux^2 uy,  k_111 = -ux uy uz,
+//   k_220 = 3 ux^2 uy^2 + s_xx s_yy + 2 s_xy^2,
+//   k_211 = 3 ux^2 uy uz + s_xx s_yz + 2 s_xy s_xz,
+//   k_221 = -6 ux^2 uy^2 uz + s_xx k_021 + s_yy k_201 + 4 s_xy k_111 + 2 (s_xz k_120 + s_yz k_210),
+//   k_222 = the sum over the set partitions of {x, x, y, y, z, z}   (and permutations).
+// The 16-bit forms of the D3Q27 step are bound by instruction issue: 256^3 decaying
+// turbulence, fp16 deviations, 395 us per step by geier27, 308 us here (5.9 TB/s).
+// kDev: f holds the deviations f - w_q on entry and on return.  Density and stress are
+// then sums of deviations (d_xx = m_xx - (rho - 1) / 3 - rho ux^2), and the weights'
+// eight nonzero raw moments are taken off before the inverse sweeps.
+template <typename C, bool kDev>
+__device__ __forceinline__ void geier27_unit(C (&f)[27], bool eq_floor, C omega) {
+  const auto P = [&](int x, int y, int z) -> C& { return f[f27::IDX.pop[x][y][z]]; };
+  // moments up to second order: x sweep, then the y and z sums that are needed
+  C g0[3][3], g1[3][3], g2[3][3];
+#pragma unroll
+  for (int y = 0; y < 3; ++y)
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+      g2[y][z] = P(2, y, z) + P(0, y, z);
+      g1[y][z] = P(2, y, z) - P(0, y, z);
+      g0[y][z] = g2[y][z] + P(1, y, z);
+    }
+  C h00[3], h01[3], h02[3], h10[3], h11[3], h20[3];
+#pragma unroll
+  for (int z = 0; z < 3; ++z) {
+    h02[z] = g0[2][z] + g0[0][z];
+    h01[z] = g0[2][z] - g0[0][z];
+    h00[z] = h02[z] + g0[1][z];
+    h11[z] = g1[2][z] - g1[0][z];
+    h10[z] = (g1[2][z] + g1[0][z]) + g1[1][z];
+    h20[z] = (g2[2][z] + g2[0][z]) + g2[1][z];
+  }
+  const auto sum3 = [](const C (&h)[3]) { return (h[2] + h[0]) + h[1]; };
+  const C m002 = h00[2] + h00[0];
+  const C rho_d = m002 + h00[1];  // rho, or rho - 1 in deviations
+  const C rho = kDev ? rho_d + C(1) : rho_d;
+  const C rho_safe = rho > C(1e-12) ? rho : C(1e-12);
+  const C inv = recip(rho_safe);
+  const C jx = sum3(h10), jy = sum3(h01), jz = h00[2] - h00[0];
+  const C ux = jx * inv, uy = jy * inv, uz = jz * inv;
+  // trace-free second-order cumulants, relaxed; the equilibrium's are rho / 3 and 0
+  const C ir = C(1) / rho;
+  const C third = C(1.0 / 3.0);
+  // (rho_eq differs from rho only below the density floor, where it moves the diagonal)
+  const C r3 = kDev ? rho_d * third : (eq_floor ? rho_safe : rho) * third;
+  const C rx = rho * ux, ry = rho * uy, rz = rho * uz;
+  const C dxx = sum3(h20) - r3 - rx * ux, dyy = sum3(h02) - r3 - ry * uy, dzz = m002 - r3 - rz * uz;
+  const C tr3 = (dxx + dyy + dzz) * third;
+  const C keep = (C(1) - omega) * ir;
+  const C sxx = fma(keep, dxx - tr3, third), syy = fma(keep, dyy - tr3, third), szz = fma(keep, dzz - tr3, third);
+  const C sxy = keep * (sum3(h11) - rx * uy), sxz = keep * ((h10[2] - h10[0]) - rx * uz),
+          syz = keep * ((h01[2] - h01[0]) - ry * uz);
+  // central moments per unit mass, by exponents
+  const C x2 = ux * ux, y2 = uy * uy, z2 = uz * uz, xy = ux * uy, xz = ux * uz, yz = uy * uz;
+  const C k210 = -x2 * uy, k201 = -x2 * uz, k120 = -y2 * ux, k021 = -y2 * uz, k102 = -z2 * ux, k012 = -z2 * uy;
+  const C k111 = -xy * uz;
+  const C c220 = C(3) * x2 * y2, c202 = C(3) * x2 * z2, c022 = C(3) * y2 * z2;
+  const C c211 = C(3) * x2 * yz, c121 = C(3) * y2 * xz, c112 = C(3) * z2 * xy;
+  const C two = C(2), four = C(4);
+  C k[3][3][3];
+  k[0][0][0] = C(1);
+  k[1][0][0] = k[0][1][0] = k[0][0][1] = C(0);
+  k[2][0][0] = sxx, k[0][2][0] = syy, k[0][0][2] = szz;
+  k[1][1][0] = sxy, k[1][0][1] = sxz, k[0][1][1] = syz;
+  k[2][1][0] = k210, k[2][0][1] = k201, k[1][2][0] = k120, k[0][2][1] = k021, k[1][0][2] = k102, k[0][1][2] = k012;
+  k[1][1][1] = k111;
+  k[2][2][0] = fma(sxx, syy, fma(two * sxy, sxy, c220));
+  k[2][0][2] = fma(sxx, szz, fma(two * sxz, sxz, c202));
+  k[0][2][2] = fma(syy, szz, fma(two * syz, syz, c022));
+  k[2][1][1] = fma(sxx, syz, fma(two * sxy, sxz, c211));
+  k[1][2][1] = fma(syy, sxz, fma(two * sxy, syz, c121));
+  k[1][1][2] = fma(szz, sxy, fma(two * sxz, syz, c112));
+  // c_221 = -6 ux^2 uy^2 uz = -2 c_220 uz
+  k[2][2][1] = fma(sxx, k021, fma(syy, k201, fma(four * sxy, k111, two * fma(sxz, k120, fma(syz, k210, -c220 * uz)))));
+  k[2][1][2] = fma(sxx, k012, fma(szz, k210, fma(four * sxz, k111, two * fma(sxy, k102, fma(syz, k201, -c202 * uy)))));
+  k[1][2][2] = fma(syy, k102, fma(szz, k120, fma(four * syz, k111, two * fma(sxy, k012, fma(sxz, k021, -c022 * ux)))));
+  // pairs with a fourth-order cumulant, two third-order ones (4 k_111^2 + 2 (k_210 k_012 +
+  // k_201 k_021 + k_120 k_102) = 10 k_111^2), three pairs; C_222 of the equilibrium is 0
+  const C pairs4 = fma(sxx, c022, fma(syy, c202, szz * c220));
+  const C mixed4 = fma(sxy, c112, fma(sxz, c121, syz * c211));
+  const C triple = fma(sxx, syz * syz, fma(syy, sxz * sxz, fma(szz, sxy * sxy, four * sxy * sxz * syz)));
+  k[2][2][2] = fma(two, triple, fma(sxx * syy, szz, fma(four, mixed4, fma(C(10) * k111, k111, pairs4))));
+  // raw moments: binomial shifts along z, y, x
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      const C m0 = k[a][b][0], m1 = k[a][b][1];
+      k[a][b][2] = fma(z2, m0, fma(two * uz, m1, k[a][b][2]));
+      k[a][b][1] = fma(uz, m0, m1);
+    }
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const C m0 = k[a][0][c], m1 = k[a][1][c];
+      k[a][2][c] = fma(y2, m0, fma(two * uy, m1, k[a][2][c]));
+      k[a][1][c] = fma(uy, m0, m1);
+    }
+  C m[27];
+#pragma unroll
+  for (int b = 0; b < 3; ++b)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const C m0 = k[0][b][c], m1 = k[1][b][c];
+      k[2][b][c] = fma(x2, m0, fma(two * ux, m1, k[2][b][c]));
+      k[1][b][c] = fma(ux, m0, m1);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const double w = f27::s3(a, b, c);  // the weights' own moment
+        if (a + b + c == 0) m[f27::IDX.mom[0][0][0]] = rho_d;  // mass and momentum as they came
+        else if (a + b + c == 1) m[f27::IDX.mom[a][b][c]] = a ? jx : (b ? jy : jz);
+        else m[f27::IDX.mom[a][b][c]] = kDev && w != 0.0 ? fma(k[a][b][c], rho, C(-w)) : k[a][b][c] * rho;
+      }
+    }
+  f27::inverse(m, f);
+}
+
 // Legacy D3Q27 "cumulant" of collide_cumulant_d3q27 (cumulant.py:935-1047):
 // central moments of f_neq pass through the pseudo-cumulant map of
 // cumulant.py:470-577 (Geier's partition terms without 1/rho; orders <= 3

@@ -51,6 +51,10 @@ enum Feat {
   FEAT_MLP_ALL = FEAT_MLP | FEAT_ALL
 };
 
+// TLBM_COLL_GEIER with the constant tau mode and omega_b = omega_odd = omega_even = 1
+// (geier27_unit); chosen by run_store, never seen at the interface
+constexpr int COLL_GEIER_UNIT = 16;
+
 // boundary kind known at compile time (a TLBM_BC_* value) or read from the launch
 constexpr int BCK_RUNTIME = -1;
 
@@ -196,14 +200,19 @@ __device__ __forceinline__ void own_force_sample(const KArgs<typename Store<S>::
 // collision (the closure kernel issues its next plane's loads there).
 // The BGK collision of the deviation storage forms hands back f - w (the
 // relaxation absorbs the shift), so their stores convert only; every other
-// collision, and streaming alone, hands back f.
-template <int S, int COLL>
-constexpr bool dev_out() {
-  return Store<S>::kDev && COLL == TLBM_COLL_BGK;
+// collision, and streaming alone, hands back f.  geier27_unit takes and hands back
+// f - w where nothing stands between the loads and it (no mask, no boundary).
+template <int S, int COLL, int FEAT>
+constexpr bool dev_in() {
+  return Store<S>::kDev && COLL == COLL_GEIER_UNIT && (FEAT & FEAT_BC) == 0;
 }
-template <class L, int S, int COLL>
+template <int S, int COLL, int FEAT>
+constexpr bool dev_out() {
+  return Store<S>::kDev && (COLL == TLBM_COLL_BGK || dev_in<S, COLL, FEAT>());
+}
+template <class L, int S, int COLL, int FEAT>
 __device__ __forceinline__ typename Store<S>::T put_out(typename Store<S>::C v, int q) {
-  if constexpr (dev_out<S, COLL>()) return Store<S>::put_dev(v);
+  if constexpr (dev_out<S, COLL, FEAT>()) return Store<S>::put_dev(v);
   else return Store<S>::template put<L>(v, q);
 }
 
@@ -211,7 +220,7 @@ struct NoHook {
   __device__ void operator()() const {}
 };
 // kDevIn: f (and what `pulled` returns) holds the deviations f - w_q of a 16-bit
-// deviation store through to the collision; the closure march's BGK step only.
+// deviation store through to the collision; the closure march's BGK step and dev_in().
 template <class L, int S, int COLL, bool STREAM, int FEAT, int BCN, int BCK, bool kDevIn = false, class Pulled,
           class EqUnit, class Blob = const mlp::Packed*, class Hook = NoHook>
 __device__ __forceinline__ void update_cell(typename Store<S>::C (&f)[L::Q], const KArgs<typename Store<S>::C>& a,
@@ -224,7 +233,8 @@ __device__ __forceinline__ void update_cell(typename Store<S>::C (&f)[L::Q], con
   constexpr bool kAll = (FEAT & FEAT_BC) != 0;
   constexpr bool kForce = (FEAT & FEAT_FORCE) != 0;
   constexpr bool kMlp = (FEAT & FEAT_MLP) != 0;
-  static_assert(!kDevIn || (dev_out<S, COLL>() && kMlp), "deviations through the closure's BGK step only");
+  static_assert(!kDevIn || (dev_out<S, COLL, FEAT>() && (kMlp || dev_in<S, COLL, FEAT>())),
+                "deviations through the closure's BGK step and the unit-rate cumulants only");
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   // a compile-time kind folds the other boundaries away
   const int bck = BCK == BCK_RUNTIME ? a.bc_kind : BCK;
@@ -330,7 +340,9 @@ __device__ __forceinline__ void update_cell(typename Store<S>::C (&f)[L::Q], con
   }
   before_collision();
 
-  if constexpr (COLL != TLBM_COLL_NONE) {
+  if constexpr (COLL == COLL_GEIER_UNIT) {
+    if constexpr (Q == 27) geier27_unit<C, kDevIn>(f, a.eq_floor != 0, a.omega);
+  } else if constexpr (COLL != TLBM_COLL_NONE) {
     const Macro<C> mc = macro<L, C, kDevIn>(f);
     const C rho_eq = a.eq_floor ? mc.rho_safe : mc.rho;
     C omega = a.omega;
@@ -368,7 +380,7 @@ __device__ __forceinline__ void update_cell(typename Store<S>::C (&f)[L::Q], con
       // tau_eff = tau + 3 nu_t, floored at 0.5 + 1e-3 (ai/inference.py:56-65)
       C te = a.tau + C(3) * C(nu);
       te = te < C(0.501) ? C(0.501) : te;
-      bgk_relax<L, C, dev_out<S, COLL>(), kDevIn>(f, rho_eq, mc.ux, mc.uy, mc.uz, approx_rcp(te));
+      bgk_relax<L, C, dev_out<S, COLL, FEAT>(), kDevIn>(f, rho_eq, mc.ux, mc.uy, mc.uz, approx_rcp(te));
     } else if constexpr (COLL == TLBM_COLL_BGK) {
       if (need_pi) {
         C feq[Q], fneq[Q], pi[6];
@@ -385,7 +397,7 @@ __device__ __forceinline__ void update_cell(typename Store<S>::C (&f)[L::Q], con
       if constexpr (!STREAM) {
         if (a.tau_mode == TLBM_TAU_FIELD64) omega = C(1) / C(reinterpret_cast<const double*>(a.tau_eff)[cell]);
       }
-      bgk_relax<L, C, dev_out<S, COLL>()>(f, rho_eq, mc.ux, mc.uy, mc.uz, omega);
+      bgk_relax<L, C, dev_out<S, COLL, FEAT>()>(f, rho_eq, mc.ux, mc.uy, mc.uz, omega);
     } else {
       // the Geier collision takes the equilibrium's moments in closed form and the
       // LES stress from the moments of f, so it never forms f_eq
@@ -428,8 +440,15 @@ __device__ __forceinline__ void update_cell(typename Store<S>::C (&f)[L::Q], con
 
 }
 
+// a stored value as the kernel carries it: f, or the deviation itself
+template <class L, int S, bool Dev>
+__device__ __forceinline__ typename Store<S>::C take(typename Store<S>::T v, int q) {
+  if constexpr (Dev) return Store<S>::get_dev(v);
+  else return Store<S>::template get<L>(v, q);
+}
+
 // Q pulled populations of cell (x, y, z) from the input lattice (periodic wrap)
-template <class L, int S>
+template <class L, int S, bool Dev = false>
 __device__ __forceinline__ void gather(typename Store<S>::C (&f)[L::Q], const typename Store<S>::T* fin,
                                        const KArgs<typename Store<S>::C>& a, int x, int y, int z) {
   using ST = Store<S>;
@@ -442,7 +461,7 @@ __device__ __forceinline__ void gather(typename Store<S>::C (&f)[L::Q], const ty
     const int sy = src_of(L::cy[q], yd, y, yu);
     const int sz = src_of(L::cz[q], zd, z, zu);
     const typename ST::T* base = fin + int64_t(q) * a.isq + int64_t(sz) * a.isz;
-    f[q] = ST::template get<L>(ld_off(base, uint32_t(sy) * uint32_t(a.isy) + uint32_t(sx)), q);
+    f[q] = take<L, S, Dev>(ld_off(base, uint32_t(sy) * uint32_t(a.isy) + uint32_t(sx)), q);
   }
 }
 
@@ -499,6 +518,7 @@ __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
   using C = typename ST::C;
   constexpr int Q = L::Q;
   constexpr bool kAll = (FEAT & FEAT_BC) != 0;
+  constexpr bool kDevIn = dev_in<S, COLL, FEAT>();
 
   const uint32_t tile = blockIdx.x;
   const uint32_t txi = tile % uint32_t(a.tiles_x);
@@ -517,7 +537,7 @@ __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
 
   C f[Q];
   if constexpr (STREAM) {
-    gather<L, S>(f, fin, a, xx, yy, z);
+    gather<L, S, kDevIn>(f, fin, a, xx, yy, z);
   } else {
     const uint32_t off = uint32_t(yy) * uint32_t(a.isy) + uint32_t(xx);
 #pragma unroll
@@ -552,13 +572,13 @@ __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
     return pull_one<ST, L>(fin, a, q, px, py, pz);
   };
   auto eq_unit = [&](C (&e)[Q]) { equilibrium_here<L>(C(1), a.bc_u, e); };
-  update_cell<L, S, COLL, STREAM, FEAT, BCN_PULL, BCK>(f, a, xx, yy, z, cell, solid, false, fx, fy, fz, pulled,
-                                                        eq_unit);
+  update_cell<L, S, COLL, STREAM, FEAT, BCN_PULL, BCK, kDevIn>(f, a, xx, yy, z, cell, solid, false, fx, fy, fz,
+                                                               pulled, eq_unit);
   if (active) {
     T* fout = static_cast<T*>(a.fout);
     const uint32_t off = uint32_t(yy) * uint32_t(a.osy) + uint32_t(xx);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, put_out<L, S, COLL>(f[q], q));
+    for (int q = 0; q < Q; ++q) st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, put_out<L, S, COLL, FEAT>(f[q], q));
   }
   if constexpr ((FEAT & FEAT_FORCE) != 0) {
     if (a.force != nullptr) force_flush(a.force, fx, fy, fz, solid);
@@ -658,6 +678,7 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
   using C = typename ST::C;
   constexpr int Q = L::Q;
   constexpr int EC = tile2_cells<L, S>();
+  constexpr bool kDevIn = dev_in<S, COLL, FEAT>();
   // The tile is a launch parameter: 64 x 8 where rows are whole cache lines, else the
   // shape that wastes fewest lanes on this grid (plan2).  The LDS rows keep a fixed
   // pitch of EC cells, so a run-time tile costs three more address registers than a
@@ -747,7 +768,7 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
     } else if constexpr (kAll) {
       if (a.solid != nullptr) pre_mask = a.solid[(uint32_t(pz) * uint32_t(ny) + uint32_t(gy)) * uint32_t(nx) + uint32_t(gx)];
     }
-    gather<L, S>(pre, fin, a, gxn, gy, pz);
+    gather<L, S, kDevIn>(pre, fin, a, gxn, gy, pz);
   };
   // first row of the set holding population q, for the plane written j-th in the march
   auto set_row = [](int cz, int j) {
@@ -764,7 +785,7 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
     const bool solid = pre_mask != 0;
     if constexpr (kForce) {
       double sx = 0.0, sy = 0.0, sz = 0.0;
-      update_cell<L, S, COLL, true, FEAT, BCN_IN_F, BCK>(f, a, gx, gy, pz, cell, solid, nb_edge, sx, sy, sz, unused,
+      update_cell<L, S, COLL, true, FEAT, BCN_IN_F, BCK, kDevIn>(f, a, gx, gy, pz, cell, solid, nb_edge, sx, sy, sz, unused,
                                                          eq_unit);
       if (own1 && solid && p >= z0 && p < zend) {
         fx += sx;
@@ -773,14 +794,14 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
         sampled = true;
       }
     } else {
-      update_cell<L, S, COLL, true, FEAT, BCN_IN_F, BCK>(f, a, gx, gy, pz, cell, solid, nb_edge, unused_force,
+      update_cell<L, S, COLL, true, FEAT, BCN_IN_F, BCK, kDevIn>(f, a, gx, gy, pz, cell, solid, nb_edge, unused_force,
                                                          unused_force, unused_force, unused, eq_unit);
     }
     const int row_a = set_row(-1, j), row_b = set_row(0, j), row_c = set_row(1, j);
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       const int row = (L::cz[q] < 0 ? row_a : L::cz[q] == 0 ? row_b : row_c) + R::index(q);
-      s[row * EC + t] = put_out<L, S, COLL>(f[q], q);
+      s[row * EC + t] = put_out<L, S, COLL, FEAT>(f[q], q);
     }
     if constexpr (kAll) s_solid[(j % 3) * EC + t] = solid ? 1 : 0;
   };
@@ -822,7 +843,7 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
       auto lds_at = [&](int q, int x, int, int) -> C {  // only ever for this lane's y
         const int row = (L::cz[q] < 0 ? row_a : L::cz[q] == 0 ? row_b : row_c) + R::index(q);
         const int at = L::cy[q] == 0 ? at_0 : (L::cy[q] > 0 ? at_p : at_m);
-        return ST::template get<L>(s[row * EC + at + (x - ux_) - L::cx[q]], q);
+        return take<L, S, kDevIn>(s[row * EC + at + (x - ux_) - L::cx[q]], q);
       };
       C f[Q];
 #pragma unroll
@@ -832,7 +853,7 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
       if constexpr (kAll) solid = s_solid[((k + 1) % 3) * EC + at_0] != 0;
       if constexpr (kForce) {
         double sx = 0.0, sy = 0.0, sz = 0.0;
-        update_cell<L, S, COLL, true, FEAT, BCN_PULL, BCK>(f, a, ux_, uy_, z, cell, solid, false, sx, sy, sz, lds_at,
+        update_cell<L, S, COLL, true, FEAT, BCN_PULL, BCK, kDevIn>(f, a, ux_, uy_, z, cell, solid, false, sx, sy, sz, lds_at,
                                                            eq_unit);
         if (own && solid) {
           fx += sx;
@@ -841,7 +862,7 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
           sampled = true;
         }
       } else {
-        update_cell<L, S, COLL, true, FEAT, BCN_PULL, BCK>(f, a, ux_, uy_, z, cell, solid, false, unused_force,
+        update_cell<L, S, COLL, true, FEAT, BCN_PULL, BCK, kDevIn>(f, a, ux_, uy_, z, cell, solid, false, unused_force,
                                                            unused_force, unused_force, lds_at, eq_unit);
       }
       T* fout = static_cast<T*>(a.fout);
@@ -851,7 +872,7 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
       T o[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        o[q] = put_out<L, S, COLL>(f[q], q);
+        o[q] = put_out<L, S, COLL, FEAT>(f[q], q);
         asm volatile("" : "+v"(o[q]));
       }
       if (own) {
@@ -901,7 +922,7 @@ __device__ __forceinline__ void lbm_mlp_body(const KArgs<typename Store<S>::C>& 
   constexpr bool kAll = (FEAT & FEAT_BC) != 0;
   // with 16-bit deviation storage the step runs in f - w from load to store: the
   // loads skip adding w_q and the collision folds it into one term per cell
-  constexpr bool kDevIn = dev_out<S, COLL>() && (FEAT & FEAT_MLP) != 0;
+  constexpr bool kDevIn = dev_out<S, COLL, FEAT>() && (FEAT & FEAT_MLP) != 0;
   __shared__ mlp::Packed s_blob;
   // f_eq(rho = 1, bc_u) for the inlet and the far-field faces, formed once per
   // workgroup instead of by every wave with such a lane on every plane, and its
@@ -1044,7 +1065,7 @@ __device__ __forceinline__ void lbm_mlp_body(const KArgs<typename Store<S>::C>& 
     asm volatile("" : "+v"(offl));
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-      st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, offl, put_out<L, S, COLL>(f[q], q));
+      st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, offl, put_out<L, S, COLL, FEAT>(f[q], q));
   }
   if constexpr ((FEAT & FEAT_FORCE) != 0) {
     if (a.force != nullptr)
@@ -2037,7 +2058,7 @@ constexpr bool coll_built() {
   if (COLL == TLBM_COLL_NONE || COLL == TLBM_COLL_BGK || COLL == TLBM_COLL_MRT) return true;
   if (COLL == TLBM_COLL_CM) return true;
   if (COLL == TLBM_COLL_CUMULANT) return L::Q != 9;
-  if (COLL == TLBM_COLL_GEIER) return L::Q == 27;
+  if (COLL == TLBM_COLL_GEIER || COLL == COLL_GEIER_UNIT) return L::Q == 27;
   return false;
 }
 
@@ -2141,6 +2162,11 @@ int run_store(const Call& c) {
     case TLBM_COLL_CUMULANT:
       return run_coll<L, S, TLBM_COLL_CUMULANT>(c);
     case TLBM_COLL_GEIER:
+      if constexpr (L::Q == 27) {
+        const tlbm_collision& k = *c.coll;
+        if (k.tau_mode == TLBM_TAU_CONST && k.rate[0] == 1.0 && k.rate[1] == 1.0 && k.rate[2] == 1.0)
+          return run_coll<L, S, COLL_GEIER_UNIT>(c);
+      }
       return run_coll<L, S, TLBM_COLL_GEIER>(c);
     default:
       return fail(TLBM_ERR_INVALID, "unknown collision kind %d", c.kind);
