@@ -1073,10 +1073,19 @@ __device__ __forceinline__ void lbm_mlp_body(const KArgs<typename Store<S>::C>& 
   }
 }
 
-// planes marched per workgroup by the learned-closure step
-#ifndef TLBM_MLP_ZPER
-#define TLBM_MLP_ZPER 16
-#endif
+// Planes marched per workgroup by the learned-closure step, for `cols` column tiles of
+// nz planes.  A longer march hides more of the loads and stages the blob less often, but
+// 1024 workgroups fill the chip (four to a CU) and a few rounds of them are needed for
+// the last one not to idle it: the march that leaves four rounds, at most 16 planes.
+// 256^3: 16 (279 us; 305 marching 4).  Smaller grids marched 16 planes with most
+// CUs idle: fp16 deviations, 150 x 130 x 100 78 -> 53 us, 180 x 170 x 160 146 -> 124 us,
+// 90 x 60 x 60 39.7 -> 14.1 us, 65 x 50 x 40 80.7 -> 12.5 us (192^3: 9 or 16 planes alike).
+inline int mlp_zper(uint64_t cols, int nz) {
+  const double x = double(cols) * nz / 4096.0;
+  if (x < 0.25) return 1;
+  const int z = int(x + 0.5);
+  return z < 2 ? 2 : (z > 16 ? 16 : z);
+}
 
 // The march pays where the step is bound by instruction issue, i.e. with 16-bit
 // storage (256^3 channel + sphere, fp16 deviations, one box: 43.9 GLUPS one cell
@@ -1717,9 +1726,10 @@ int fill_args(KArgs<C>& a, int lattice, const void* fin, const int64_t* is, void
 template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK = BCK_RUNTIME>
 int launch_lbm(const KArgs<typename Store<S>::C>& a, int bx, int by, uint32_t nb, hipStream_t s) {
   if constexpr ((FEAT & FEAT_MLP) != 0) {
-    // nb = tiles_x * tiles_y * nz; the closure step marches TLBM_MLP_ZPER planes per workgroup
-    const int zper = mlp_marches<S>() ? TLBM_MLP_ZPER : 1;
-    const uint32_t nbz = uint32_t(a.tiles_x) * uint32_t(a.tiles_y) * uint32_t((a.nz + zper - 1) / zper);
+    // nb = tiles_x * tiles_y * nz; the closure step marches zper planes per workgroup
+    const uint32_t cols = uint32_t(a.tiles_x) * uint32_t(a.tiles_y);
+    const int zper = mlp_marches<S>() ? mlp_zper(cols, a.nz) : 1;
+    const uint32_t nbz = cols * uint32_t((a.nz + zper - 1) / zper);
     (void)nb;
     hipLaunchKernelGGL((k_lbm_mlp<L, S, COLL, STREAM, FEAT, BCK>), dim3(nbz), dim3(bx, by), 0, s, a, zper);
   } else {
