@@ -70,6 +70,7 @@ struct KArgs {
   int64_t osq, osz, osy;  // output strides
   int nx, ny, nz, tiles_x, tiles_y;
   int tau_mode, eq_floor, bc_kind, bc_faces;
+  uint32_t row_mul, row_shift;  // flat tiles: c / nx = umulhi(c, row_mul) >> row_shift; row_mul 0: tiles of rows
   C omega, tau, cs_delta_sq, tau_cap;
   C rate[8];
   C bc_u[3];
@@ -511,6 +512,14 @@ __device__ __forceinline__ bool take_neighbour(int bck, int faces, int x, int nx
   return false;
 }
 
+// Whether the one-step kernel may take 256 consecutive cells of a plane instead of a
+// tile of rows: the inlet / outlet lane permute (mask and boundary kernels without a
+// force buffer) needs whole waves along x.
+template <bool STREAM, int FEAT>
+constexpr bool flat_tiles() {
+  return (FEAT & FEAT_MLP) == 0 && (!STREAM || (FEAT & FEAT_BC) == 0 || (FEAT & FEAT_FORCE) != 0);
+}
+
 template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK>
 __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
   using ST = Store<S>;
@@ -521,13 +530,24 @@ __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
   constexpr bool kDevIn = dev_in<S, COLL, FEAT>();
 
   const uint32_t tile = blockIdx.x;
-  const uint32_t txi = tile % uint32_t(a.tiles_x);
-  const uint32_t rest = tile / uint32_t(a.tiles_x);
-  const uint32_t tyi = rest % uint32_t(a.tiles_y);
-  const int z = int(rest / uint32_t(a.tiles_y));
-  const int x = int(txi * blockDim.x + threadIdx.x);
-  const int y = int(tyi * blockDim.y + threadIdx.y);
-  const bool active = x < a.nx && y < a.ny;
+  int x, y, z;
+  bool active;
+  if (flat_tiles<STREAM, FEAT>() && a.row_mul != 0) {
+    // 256 consecutive cells of a plane
+    z = int(tile / uint32_t(a.tiles_x));
+    const uint32_t c = (tile - uint32_t(z) * uint32_t(a.tiles_x)) * 256u + threadIdx.x;
+    y = int(__umulhi(c, a.row_mul) >> a.row_shift);
+    x = int(c) - y * a.nx;
+    active = y < a.ny;
+  } else {
+    const uint32_t txi = tile % uint32_t(a.tiles_x);
+    const uint32_t rest = tile / uint32_t(a.tiles_x);
+    const uint32_t tyi = rest % uint32_t(a.tiles_y);
+    z = int(rest / uint32_t(a.tiles_y));
+    x = int(txi * blockDim.x + threadIdx.x);
+    y = int(tyi * blockDim.y + threadIdx.y);
+    active = x < a.nx && y < a.ny;
+  }
   if (FEAT == FEAT_NONE && !active) return;
   // inactive lanes (force / closure paths) work on cell (0, 0, z): in bounds, never stored
   const int xx = active ? x : 0;
@@ -1733,6 +1753,25 @@ int launch_lbm(const KArgs<typename Store<S>::C>& a, int bx, int by, uint32_t nb
     (void)nb;
     hipLaunchKernelGGL((k_lbm_mlp<L, S, COLL, STREAM, FEAT, BCK>), dim3(nbz), dim3(bx, by), 0, s, a, zper);
   } else {
+    // Rows that do not fill their waves: tiles of consecutive cells, y and x by one
+    // multiply.  96 x 96 x 193 with force and LES: four waves a row, the fourth with one
+    // lane, 73 us; flat, and with the boundary-free kernel below, 55.6 us.  From 1.04x idle lanes on.
+    if constexpr (flat_tiles<STREAM, FEAT>()) {
+      if (a.nx >= 2 && (a.nx + 63) / 64 * 64 > 1.04 * a.nx) {
+        KArgs<typename Store<S>::C> b = a;
+        // for c < 2^31: m = ceil(2^(31 + k) / nx), 2^k >= nx, so c m / 2^(31 + k) exceeds
+        // c / nx by less than c nx / (2^(31 + k) nx) < 1 / nx
+        int k = 1;
+        while ((int64_t(1) << k) < a.nx) ++k;
+        b.row_mul = uint32_t(((uint64_t(1) << (31 + k)) + uint64_t(a.nx) - 1) / uint64_t(a.nx));
+        b.row_shift = uint32_t(k - 1);
+        b.tiles_x = int((uint64_t(a.nx) * uint64_t(a.ny) + 255) / 256);
+        b.tiles_y = 1;
+        hipLaunchKernelGGL((k_lbm<L, S, COLL, STREAM, FEAT, BCK>), dim3(uint32_t(b.tiles_x) * uint32_t(a.nz)),
+                           dim3(256), 0, s, b);
+        return check_launch("k_lbm");
+      }
+    }
     hipLaunchKernelGGL((k_lbm<L, S, COLL, STREAM, FEAT, BCK>), dim3(nb), dim3(bx, by), 0, s, a);
   }
   return check_launch("k_lbm");
@@ -2146,6 +2185,13 @@ int run_coll(const Call& c) {
     if (c.stream_) {
       if constexpr (L::Q == 19 && COLL == TLBM_COLL_BGK) {
         if (c.feat && c.force == nullptr) return launch_lbm_kind<L, S, COLL, FEAT_BC>(a, bx, by, nb, c.s);
+      }
+      // the obstacle step (force, no face condition; triton_fused_obstacle.py:1695-2053): the
+      // state of the boundary kinds it never has spilled 23 scalar registers
+      if constexpr (L::Q == 19 && (S == ST_F32 || S == ST_F64) &&
+                    (COLL == TLBM_COLL_BGK || COLL == TLBM_COLL_CM || COLL == TLBM_COLL_CUMULANT)) {
+        if (c.force != nullptr && a.bc_kind == TLBM_BC_NONE)
+          return launch_lbm<L, S, COLL, true, FEAT_ALL, TLBM_BC_NONE>(a, bx, by, nb, c.s);
       }
       if (c.feat) return launch_lbm<L, S, COLL, true, FEAT_ALL>(a, bx, by, nb, c.s);
       return launch_lbm<L, S, COLL, true, FEAT_NONE>(a, bx, by, nb, c.s);
