@@ -420,9 +420,12 @@ typedef struct tlbm_cavity {
 /* host only: fill offset / tiles_before from the edges; totals in elements and tiles */
 int tlbm_cavities_layout(tlbm_cavity* cavs, int n, int64_t* total_elements, int64_t* total_tiles);
 
-/* one step of every cavity, f_in -> f_out (distinct buffers of `capacity` elements; store
+/* tlbm_cavities_fill: every cavity at rest, rho = 1 (f_q = w_q; 0 in deviation storage), the padding
+ * untouched.
+ * tlbm_cavities_step: one step of every cavity, f_in -> f_out (distinct buffers of `capacity` elements; store
  * F32, F64, F16_DEV or BF16_DEV).  grid = 0: one workgroup per tile; grid > 0: a persistent
  * grid of that many workgroups striding over the tiles. */
+int tlbm_cavities_fill(int store, void* f, int64_t capacity, const tlbm_cavity* cavs, int n, tlbm_stream_t stream);
 int tlbm_cavities_step(int store, const void* f_in, void* f_out, int64_t capacity, const tlbm_cavity* cavs,
                        int n, double u_lid, int grid, tlbm_stream_t stream);
 

@@ -144,6 +144,7 @@ _SIGNATURES = {
     "tlbm_coarsen_moments": ([_I, _I, _VP, _VP, _I, _I, _I, _I, _VP, _VP], _I),
     "tlbm_sgs_samples": ([_VP, _I, _I, _I, _VP, _VP, _VP], _I),
     "tlbm_cavities_layout": ([_VP, _I, _VP, _VP], _I),
+    "tlbm_cavities_fill": ([_I, _VP, _I64, _VP, _I, _VP], _I),
     "tlbm_cavities_step": ([_I, _VP, _VP, _I64, _VP, _I, ctypes.c_double, _I, _VP], _I),
     "tlbm_cavities_graph": ([_I, _VP, _VP, _I64, _VP, _I, ctypes.c_double, _I, _I, _VP], _I),
     "tlbm_cavities_step2": ([_I, _VP, _VP, _I64, _VP, _I, ctypes.c_double, _I, _VP], _I),
