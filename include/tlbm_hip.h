@@ -157,6 +157,17 @@ int tlbm_step2(int lattice, int store, const void* f_in, const int64_t* in_strid
                const int64_t* out_strides, int nz, int ny, int nx, const tlbm_collision* coll,
                const int8_t* solid, const tlbm_boundary* bc, double* force, tlbm_stream_t stream);
 
+/*
+ * n_steps steps without a host call between them (the reporter-free run() loop,
+ * src/tensorlbm/triton_fused.py:892-895): f_in -> one of two buffers (strides buf_strides, not f_in
+ * unless it is one of them) -> the other -> ..., never writing into its input: the first output is
+ * buf_b if f_in is buf_a, else buf_a.  pairs: two steps per launch (tlbm_step2), an odd last step alone.
+ * *last: 0 if the result is in buf_a, 1 in buf_b, -1 for no step.  Stops at the first failing launch.
+ */
+int tlbm_run(int lattice, int store, const void* f_in, const int64_t* in_strides, void* buf_a, void* buf_b,
+             const int64_t* buf_strides, int nz, int ny, int nx, const tlbm_collision* coll, const int8_t* solid,
+             const tlbm_boundary* bc, int n_steps, int pairs, int* last, tlbm_stream_t stream);
+
 /* 1 if tlbm_step2() serves these arguments, else 0; sets no error */
 int tlbm_step2_supported(int lattice, int store, const tlbm_collision* coll, const tlbm_boundary* bc,
                          int nx);

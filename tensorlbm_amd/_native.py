@@ -8,6 +8,7 @@ object is missing or a call fails, an exception names the problem.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from pathlib import Path
 
@@ -104,6 +105,8 @@ _SIGNATURES = {
                    ctypes.POINTER(Boundary), _VP, _VP], _I),
     "tlbm_step2": ([_I, _I, _VP, _VP, _VP, _VP, _I, _I, _I, ctypes.POINTER(Collision), _VP,
                     ctypes.POINTER(Boundary), _VP, _VP], _I),
+    "tlbm_run": ([_I, _I, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, ctypes.POINTER(Collision), _VP,
+                  ctypes.POINTER(Boundary), _I, _I, ctypes.POINTER(_I), _VP], _I),
     "tlbm_step2_supported": ([_I, _I, ctypes.POINTER(Collision), ctypes.POINTER(Boundary), _I], _I),
     "tlbm_stream": ([_I, _I, _VP, _VP, _VP, _VP, _I, _I, _I, _VP], _I),
     "tlbm_collide": ([_I, _I, _VP, _VP, _VP, _VP, _I, _I, _I, ctypes.POINTER(Collision), _VP], _I),
@@ -224,8 +227,14 @@ def strides_of(f: torch.Tensor) -> "Strides":
     return Strides(f.stride(0), f.stride(1), f.stride(2))
 
 
+# torch's current stream as a plain number, without the Stream object around it (1.6 us a call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
     """Raw hipStream_t of torch's current stream on the tensor's device."""
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
@@ -280,6 +289,14 @@ def make_collision(
     c.tau_eff = ptr(tau_eff)
     c.mlp = mlp
     return c
+
+
+@functools.lru_cache(maxsize=512)
+def shared_collision(kind: int, tau: float, tau_mode: int, eq_rho_floor: bool, cs_delta_sq: float,
+                     rates: tuple) -> Collision:
+    """One read-only parameter struct per set of values: filling a new one costs as much as the launch."""
+    return make_collision(kind, tau, tau_mode=tau_mode, eq_rho_floor=eq_rho_floor, cs_delta_sq=cs_delta_sq,
+                          rates=rates)
 
 
 def make_boundary(kind: int = BC_NONE, u=(0.0, 0.0, 0.0), faces: int = 0) -> Boundary:

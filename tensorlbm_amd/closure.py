@@ -276,20 +276,25 @@ def train_eddy_viscosity_model_3d(features: torch.Tensor, targets: torch.Tensor,
     val_idx, tr_idx = perm[:n_val], perm[n_val:]
     x_tr, y_tr = x.index_select(0, tr_idx).contiguous(), y.index_select(0, tr_idx).contiguous()
     x_val, y_val = x.index_select(0, val_idx).contiguous(), y.index_select(0, val_idx).contiguous()
+    mean, std = x_tr.mean(dim=0), x_tr.std(dim=0, unbiased=False)
+    # each epoch's order is drawn on the CPU while the GPU still works on what came before it
+    n_tr = int(x_tr.shape[0])
+    epochs = int(cfg.epochs)
+    order = torch.randperm(n_tr, generator=gen) if epochs > 0 else None
     if model is None:
         model = EddyViscosityMLP3D(device, seed=int(cfg.seed))
-    model.set_feature_stats(x_tr.mean(dim=0).cpu(), x_tr.std(dim=0, unbiased=False).cpu())
-    n_tr = int(x_tr.shape[0])
+    model.set_feature_stats(mean.cpu(), std.cpu())
     bs = max(1, min(int(cfg.batch_size), n_tr))
     opt = _Adam(model, cfg.learning_rate, clip_norm=cfg.gradient_clip_norm, max_batch=bs)
     history: list[dict] = []
     best = (float("inf"), model.params.clone(), 0)
     stale = 0
     t0 = time.perf_counter()
-    for epoch in range(int(cfg.epochs)):
-        order = torch.randperm(n_tr, generator=gen).to(device)
-        ep_loss = opt.epoch(x_tr, y_tr, order, bs)
+    for epoch in range(epochs):
+        ep_loss = opt.epoch(x_tr, y_tr, order.to(device), bs)
         pred = model(x_val).reshape(-1)
+        if epoch + 1 < epochs:
+            order = torch.randperm(n_tr, generator=gen)
         val_mse = float(torch.mean((pred - y_val) ** 2))
         met = {"epoch": epoch, "train_mse": float(ep_loss) / n_tr, "val_mse": val_mse,
                "val_mae": float(torch.mean(torch.abs(pred - y_val))), "val_r2": _r2(pred, y_val)}

@@ -2388,6 +2388,31 @@ int tlbm_step2(int lattice, int store, const void* f_in, const int64_t* in_strid
   return run(c);
 }
 
+int tlbm_run(int lattice, int store, const void* f_in, const int64_t* in_strides, void* buf_a, void* buf_b,
+             const int64_t* buf_strides, int nz, int ny, int nx, const tlbm_collision* coll, const int8_t* solid,
+             const tlbm_boundary* bc, int n_steps, int pairs, int* last, tlbm_stream_t stream) {
+  g_err[0] = 0;
+  if (n_steps < 0) return fail(TLBM_ERR_INVALID, "negative step count");
+  if (!buf_a || !buf_b || !last) return fail(TLBM_ERR_INVALID, "null pointer");
+  if (buf_a == buf_b) return fail(TLBM_ERR_ALIAS, "the two buffers alias");
+  *last = -1;
+  const void* in = f_in;
+  const int64_t* is = in_strides;
+  for (int k = 0; k < n_steps;) {
+    const int to = in == buf_a ? 1 : 0;
+    void* out = to ? buf_b : buf_a;
+    const bool two = pairs && n_steps - k >= 2;
+    const int rc = two ? tlbm_step2(lattice, store, in, is, out, buf_strides, nz, ny, nx, coll, solid, bc, nullptr, stream)
+                       : tlbm_step(lattice, store, in, is, out, buf_strides, nz, ny, nx, coll, solid, bc, nullptr, stream);
+    if (rc != TLBM_OK) return rc;
+    *last = to;
+    in = out;
+    is = buf_strides;
+    k += two ? 2 : 1;
+  }
+  return TLBM_OK;
+}
+
 int tlbm_step2_supported(int lattice, int store, const tlbm_collision* coll, const tlbm_boundary* bc, int nx) {
   return step2_reason(lattice, store, coll, bc, nx) == nullptr ? 1 : 0;
 }

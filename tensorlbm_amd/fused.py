@@ -484,7 +484,12 @@ class FusedSolver3D:
         """Advance ``n_steps``; reporters receive a StepContext after every step (lbm_step.py:615-686)."""
         if not reporters:
             n = int(n_steps)
-            if self._two_step:
+            if getattr(self.step, "__func__", None) is FusedSolver3D.step and \
+                    getattr(self.step2, "__func__", None) is FusedSolver3D.step2:
+                # whole calls of launches; short enough that an interrupt is heard
+                for k in range(0, n, 1024):
+                    f = self._run(f, min(1024, n - k))
+            elif self._two_step:
                 for _ in range(n // 2):
                     f = self.step2(f)
                 if n % 2:
@@ -493,7 +498,7 @@ class FusedSolver3D:
                 for _ in range(n):
                     f = self.step(f)
             self._report_step += n
-            return f, [{} for _ in range(int(n_steps))]
+            return f, [{} for _ in range(n)]
         from .reporters import StepContext, dispatch
 
         ctx = StepContext(step=self._report_step, f=f, lattice=self.lattice,
@@ -510,6 +515,24 @@ class FusedSolver3D:
                 break
         self._report_step = step
         return f, diags
+
+    def _run(self, f: torch.Tensor, n: int) -> torch.Tensor:
+        """``n`` steps in one library call: the launches of ``step()`` / ``step2()`` in their order and buffers."""
+        self._check_input(f)
+        self._target(f, None)
+        if self.closure is not None:
+            self._coll.mlp = self.closure.packed.data_ptr()
+        nat.require_gpu(f, "FusedSolver3D.run")
+        if f.stride(-1) != 1:
+            f = f.contiguous()
+        q, nz, ny, nx = _dims(f)
+        a, b = self._buf_a, self._buf_b
+        last = ctypes.c_int(-1)
+        rc = nat.lib().tlbm_run(q, self._store, f.data_ptr(), nat.strides_of(f), a.data_ptr(), b.data_ptr(),
+                                nat.strides_of(a), nz, ny, nx, self._coll, nat.ptr(self.solid), self._bc, n,
+                                int(self._two_step), ctypes.byref(last), nat.stream_of(f))
+        nat.check(rc, "FusedSolver3D.run")
+        return b if last.value == 1 else a
 
     def state_dict(self, f: torch.Tensor, *, step: int | None = None, extra=None) -> dict:
         """Checkpointable state of populations ``f`` (``triton_fused_state_dict``, checkpoint.py:568-586):

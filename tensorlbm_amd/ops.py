@@ -123,9 +123,8 @@ def equilibrium27(rho, ux, uy, uz, device=None, *, out=None):
 def _macroscopic(f, q, what):
     f, dims = _pops(f, q, what)
     dt = _eager_dtype(f, what)
-    spatial = tuple(f.shape[1:])
-    rho, ux, uy = (torch.empty(spatial, dtype=f.dtype, device=f.device) for _ in range(3))
-    uz = torch.empty(spatial, dtype=f.dtype, device=f.device) if q != 9 else None
+    rho, ux, uy = (torch.empty_like(f[0]) for _ in range(3))
+    uz = torch.empty_like(f[0]) if q != 9 else None
     rc = nat.lib().tlbm_macroscopic(q, dt, f.data_ptr(), rho.data_ptr(), ux.data_ptr(), uy.data_ptr(),
                                     nat.ptr(uz), dims[0] * dims[1] * dims[2], nat.stream_of(f))
     nat.check(rc, what)
@@ -162,6 +161,15 @@ def macroscopic27(f, device=None):
 # ---------------------------------------------------------------------------
 
 
+def _coll(kind, tau, *, tau_mode=nat.TAU_CONST, eq_rho_floor=False, cs_delta_sq=0.0, rates=(), tau_eff=None):
+    """Collision parameters of an eager op; shared between calls unless they point to a field."""
+    if tau_eff is None:
+        return nat.shared_collision(kind, float(tau), tau_mode, eq_rho_floor, float(cs_delta_sq),
+                                    tuple(map(float, rates)))
+    return nat.make_collision(kind, tau, tau_mode=tau_mode, eq_rho_floor=eq_rho_floor, cs_delta_sq=cs_delta_sq,
+                              rates=rates, tau_eff=tau_eff)
+
+
 def _collide(f, q, coll, what):
     f, dims = _pops(f, q, what)
     dt = _eager_dtype(f, what)
@@ -179,32 +187,32 @@ def _tau(tau, what):
 
 def collide_bgk(f, tau):
     """D2Q9 BGK ``f − (f − f_eq)/τ`` (solver.py:67-71)."""
-    return _collide(f, 9, nat.make_collision(nat.COLL_BGK, _tau(tau, "collide_bgk"), eq_rho_floor=False),
+    return _collide(f, 9, _coll(nat.COLL_BGK, _tau(tau, "collide_bgk"), eq_rho_floor=False),
                     "collide_bgk")
 
 
 def collide_bgk_fused(f, tau):
     """D2Q9 BGK in one pass (solver.py:74-117): the same update as ``collide_bgk``, one kernel here too."""
-    return _collide(f, 9, nat.make_collision(nat.COLL_BGK, _tau(tau, "collide_bgk_fused"), eq_rho_floor=False),
+    return _collide(f, 9, _coll(nat.COLL_BGK, _tau(tau, "collide_bgk_fused"), eq_rho_floor=False),
                     "collide_bgk_fused")
 
 
 def collide_bgk_matmul(f, tau):
     """D2Q9 BGK with moments by matrix products (solver.py:194-246): the same update as ``collide_bgk``;
     the moments of nine populations are a few adds per cell, no GEMM."""
-    return _collide(f, 9, nat.make_collision(nat.COLL_BGK, _tau(tau, "collide_bgk_matmul"), eq_rho_floor=False),
+    return _collide(f, 9, _coll(nat.COLL_BGK, _tau(tau, "collide_bgk_matmul"), eq_rho_floor=False),
                     "collide_bgk_matmul")
 
 
 def collide_bgk3d(f, tau):
     """D3Q19 BGK (solver3d.py:100-104)."""
-    return _collide(f, 19, nat.make_collision(nat.COLL_BGK, _tau(tau, "collide_bgk3d"), eq_rho_floor=False),
+    return _collide(f, 19, _coll(nat.COLL_BGK, _tau(tau, "collide_bgk3d"), eq_rho_floor=False),
                     "collide_bgk3d")
 
 
 def collide_bgk27(f, tau):
     """D3Q27 BGK (d3q27.py:423-435)."""
-    return _collide(f, 27, nat.make_collision(nat.COLL_BGK, _tau(tau, "collide_bgk27"), eq_rho_floor=False),
+    return _collide(f, 27, _coll(nat.COLL_BGK, _tau(tau, "collide_bgk27"), eq_rho_floor=False),
                     "collide_bgk27")
 
 
@@ -216,7 +224,7 @@ def collide_mrt(f, tau, s_e=1.64, s_eps=1.54, s_q=1.7, tau_field=None):
         if tuple(tau_field.shape) != tuple(f.shape[1:]):
             raise ValueError(f"tau_field shape {tuple(tau_field.shape)} must match {tuple(f.shape[1:])}")
         mode, te = nat.TAU_FIELD, tau_field.to(device=f.device, dtype=torch.float32).contiguous()
-    coll = nat.make_collision(nat.COLL_MRT, tau, tau_mode=mode, eq_rho_floor=False,
+    coll = _coll(nat.COLL_MRT, tau, tau_mode=mode, eq_rho_floor=False,
                               rates=(s_e, s_eps, s_q, 0.0), tau_eff=te)
     return _collide(f, 9, coll, "collide_mrt")
 
@@ -224,7 +232,7 @@ def collide_mrt(f, tau, s_e=1.64, s_eps=1.54, s_q=1.7, tau_field=None):
 def collide_mrt3d(f, tau, s_e=1.19, s_eps=1.4, s_q=1.2, s_pi=None):
     """D3Q19 MRT (solver3d.py:107-160); ``s_pi`` defaults to ``s_e``."""
     s_pi = s_e if s_pi is None else s_pi
-    coll = nat.make_collision(nat.COLL_MRT, _tau(tau, "collide_mrt3d"), eq_rho_floor=False,
+    coll = _coll(nat.COLL_MRT, _tau(tau, "collide_mrt3d"), eq_rho_floor=False,
                               rates=(s_e, s_eps, s_q, s_pi))
     return _collide(f, 19, coll, "collide_mrt3d")
 
@@ -232,7 +240,7 @@ def collide_mrt3d(f, tau, s_e=1.19, s_eps=1.4, s_q=1.2, s_pi=None):
 def collide_mrt27(f, tau, s_e=1.19, s_eps=1.4, s_q=1.2, s_pi=None):
     """D3Q27 MRT, Gram-Schmidt basis (d3q27.py:643-726)."""
     s_pi = s_e if s_pi is None else s_pi
-    coll = nat.make_collision(nat.COLL_MRT, _tau(tau, "collide_mrt27"), eq_rho_floor=False,
+    coll = _coll(nat.COLL_MRT, _tau(tau, "collide_mrt27"), eq_rho_floor=False,
                               rates=(s_e, s_eps, s_q, s_pi))
     return _collide(f, 27, coll, "collide_mrt27")
 
@@ -246,7 +254,7 @@ def collide_cumulant_d2q9(f, tau, omega_b=1.0, omega_3=1.0, omega_4=1.0):
     if f.ndim != 3 or f.shape[0] != 9:
         raise ValueError(f"D2Q9 populations must have shape (9, ny, nx), got {tuple(f.shape)}")
     tau = _tau(tau, "collide_cumulant_d2q9")
-    coll = nat.make_collision(nat.COLL_CM, tau, eq_rho_floor=False, rates=(omega_b, omega_3, omega_4))
+    coll = _coll(nat.COLL_CM, tau, eq_rho_floor=False, rates=(omega_b, omega_3, omega_4))
     return _collide(f, 9, coll, "collide_cumulant_d2q9")
 
 
@@ -257,7 +265,7 @@ def collide_cascaded_d3q19(f, tau, s_bulk=1.0, s_3=1.0, s_4=1.0):
     tau = _tau(tau, "collide_cascaded_d3q19")
     if tau <= 0.5:
         raise ValueError(f"tau must be > 0.5, got {tau}")
-    coll = nat.make_collision(nat.COLL_CM, tau, eq_rho_floor=False, rates=(s_bulk, s_3, s_4, s_4, s_4))
+    coll = _coll(nat.COLL_CM, tau, eq_rho_floor=False, rates=(s_bulk, s_3, s_4, s_4, s_4))
     return _collide(f, 19, coll, "collide_cascaded_d3q19")
 
 
@@ -270,7 +278,7 @@ def collide_cascaded_d3q27(f, tau, s_bulk=1.0, s_3=1.0, s_4=1.0, s_5=None, s_6=N
         raise ValueError(f"tau must be > 0.5, got {tau}")
     s_5 = s_4 if s_5 is None else s_5
     s_6 = s_4 if s_6 is None else s_6
-    coll = nat.make_collision(nat.COLL_CM, tau, eq_rho_floor=False, rates=(s_bulk, s_3, s_4, s_5, s_6))
+    coll = _coll(nat.COLL_CM, tau, eq_rho_floor=False, rates=(s_bulk, s_3, s_4, s_5, s_6))
     return _collide(f, 27, coll, "collide_cascaded_d3q27")
 
 
@@ -296,12 +304,12 @@ def collide_cumulant_d3q19(f, tau, omega_b=1.0, omega_odd=1.0, omega_even=1.0, C
     if C_w > 0.0 or C_v > 0.0:
         te = gradient_closure_tau(f, tau, C_w=C_w, C_v=C_v, solid_mask=solid_mask, wall_velocity=wall_velocity)
         mode = nat.TAU_FIELD64 if te.dtype == torch.float64 else nat.TAU_FIELD
-        coll = nat.make_collision(nat.COLL_CUMULANT, tau, tau_mode=mode, eq_rho_floor=False, rates=rates, tau_eff=te)
+        coll = _coll(nat.COLL_CUMULANT, tau, tau_mode=mode, eq_rho_floor=False, rates=rates, tau_eff=te)
         out = _collide(f, 19, coll, "collide_cumulant_d3q19")
         del te
         return out
     mode = nat.TAU_SMAG_RAW if C_s > 0.0 else nat.TAU_CONST
-    coll = nat.make_collision(nat.COLL_CUMULANT, tau, tau_mode=mode, eq_rho_floor=False, cs_delta_sq=C_s * C_s,
+    coll = _coll(nat.COLL_CUMULANT, tau, tau_mode=mode, eq_rho_floor=False, cs_delta_sq=C_s * C_s,
                               rates=rates)
     return _collide(f, 19, coll, "collide_cumulant_d3q19")
 
@@ -353,7 +361,7 @@ def collide_cumulant_d3q27(f, tau, omega_b=1.0, omega_odd=1.0, omega_even=1.0, C
     tau = _tau(tau, "collide_cumulant_d3q27")
     if C_s > 0:
         tau = _domain_mean_smagorinsky_tau(f, tau, C_s, "collide_cumulant_d3q27")
-    coll = nat.make_collision(nat.COLL_CUMULANT, tau, eq_rho_floor=False, rates=(omega_b, omega_odd, omega_even))
+    coll = _coll(nat.COLL_CUMULANT, tau, eq_rho_floor=False, rates=(omega_b, omega_odd, omega_even))
     return _collide(f, 27, coll, "collide_cumulant_d3q27")
 
 
@@ -378,12 +386,12 @@ def collide_cumulant_geier_d3q27(f, tau, omega_b=1.0, omega_odd=1.0, omega_even=
     tau = _tau(tau, "collide_cumulant_geier_d3q27")
     if C_s > 0.0:
         tau = _domain_mean_smagorinsky_tau(f, tau, C_s, "collide_cumulant_geier_d3q27")
-    coll = nat.make_collision(nat.COLL_GEIER, tau, eq_rho_floor=False, rates=(omega_b, omega_odd, omega_even))
+    coll = _coll(nat.COLL_GEIER, tau, eq_rho_floor=False, rates=(omega_b, omega_odd, omega_even))
     return _collide(f, 27, coll, "collide_cumulant_geier_d3q27")
 
 
 def _smag(f, q, tau, C_s, what):
-    coll = nat.make_collision(nat.COLL_BGK, _tau(tau, what), tau_mode=nat.TAU_SMAG, eq_rho_floor=False,
+    coll = _coll(nat.COLL_BGK, _tau(tau, what), tau_mode=nat.TAU_SMAG, eq_rho_floor=False,
                               cs_delta_sq=float(C_s) ** 2)
     return _collide(f, q, coll, what)
 
@@ -405,7 +413,7 @@ def collide_smagorinsky_bgk27(f, tau, C_s=0.1):
 
 def collide_smagorinsky_mrt(f, tau, C_s=0.1, s_e=1.64, s_eps=1.54, s_q=1.7):
     """D2Q9 MRT whose stress moments relax at the per-cell Smagorinsky 1/τ_eff (turbulence.py:270-342)."""
-    coll = nat.make_collision(nat.COLL_MRT, _tau(tau, "collide_smagorinsky_mrt"), tau_mode=nat.TAU_SMAG,
+    coll = _coll(nat.COLL_MRT, _tau(tau, "collide_smagorinsky_mrt"), tau_mode=nat.TAU_SMAG,
                               eq_rho_floor=False, cs_delta_sq=float(C_s) ** 2, rates=(s_e, s_eps, s_q, s_e))
     return _collide(f, 9, coll, "collide_smagorinsky_mrt")
 
@@ -413,7 +421,7 @@ def collide_smagorinsky_mrt(f, tau, C_s=0.1, s_e=1.64, s_eps=1.54, s_q=1.7):
 def collide_smagorinsky_mrt3d(f, tau, C_s=0.1, s_e=1.19, s_eps=1.4, s_q=1.2, s_pi=None):
     """D3Q19 MRT whose stress moments 9-13 relax at the per-cell Smagorinsky 1/τ_eff (turbulence.py:345-433)."""
     s_pi = s_e if s_pi is None else s_pi
-    coll = nat.make_collision(nat.COLL_MRT, _tau(tau, "collide_smagorinsky_mrt3d"), tau_mode=nat.TAU_SMAG,
+    coll = _coll(nat.COLL_MRT, _tau(tau, "collide_smagorinsky_mrt3d"), tau_mode=nat.TAU_SMAG,
                               eq_rho_floor=False, cs_delta_sq=float(C_s) ** 2, rates=(s_e, s_eps, s_q, s_pi))
     return _collide(f, 19, coll, "collide_smagorinsky_mrt3d")
 
@@ -421,7 +429,7 @@ def collide_smagorinsky_mrt3d(f, tau, C_s=0.1, s_e=1.19, s_eps=1.4, s_q=1.2, s_p
 def collide_smagorinsky_mrt27(f, tau, C_s=0.1, s_e=1.19, s_eps=1.4, s_q=1.2, s_pi=None):
     """D3Q27 MRT whose stress moments 5-9 relax at the per-cell Smagorinsky 1/τ_eff (turbulence.py:497-587)."""
     s_pi = s_e if s_pi is None else s_pi
-    coll = nat.make_collision(nat.COLL_MRT, _tau(tau, "collide_smagorinsky_mrt27"), tau_mode=nat.TAU_SMAG,
+    coll = _coll(nat.COLL_MRT, _tau(tau, "collide_smagorinsky_mrt27"), tau_mode=nat.TAU_SMAG,
                               eq_rho_floor=False, cs_delta_sq=float(C_s) ** 2, rates=(s_e, s_eps, s_q, s_pi))
     return _collide(f, 27, coll, "collide_smagorinsky_mrt27")
 
@@ -434,9 +442,10 @@ def collide_smagorinsky_mrt27(f, tau, C_s=0.1, s_e=1.19, s_eps=1.4, s_q=1.2, s_p
 def _stream(f, q, what):
     f, dims = _pops(f, q, what, contiguous=False)
     store = nat.store_code(f.dtype)
-    out = torch.empty(f.shape, dtype=f.dtype, device=f.device)
-    rc = nat.lib().tlbm_stream(q, store, f.data_ptr(), nat.strides_of(f), out.data_ptr(), None, *dims,
-                               nat.stream_of(f))
+    dense = f.is_contiguous()
+    out = torch.empty_like(f) if dense else torch.empty(f.shape, dtype=f.dtype, device=f.device)
+    rc = nat.lib().tlbm_stream(q, store, f.data_ptr(), None if dense else nat.strides_of(f), out.data_ptr(), None,
+                               *dims, nat.stream_of(f))
     nat.check(rc, what)
     return out
 
