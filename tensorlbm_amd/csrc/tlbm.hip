@@ -22,6 +22,7 @@
 // f[q] <-> f[opp(q)] of the pulled values (pull[opp q](x) = b[opp q][x + c_q]),
 // so walls cost no extra loads.
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -922,6 +923,126 @@ template <class L, int S, int COLL, int FEAT, int BCK>
 __global__ __launch_bounds__((tile2_threads<L, S>())) void k_lbm2(const KArgs<typename Store<S>::C> a,
                                                                   const Plan2 p2) {
   lbm2_body<L, S, COLL, FEAT, BCK>(a, p2, xcd_tile(blockIdx.x, gridDim.x));
+}
+
+// Two fused steps of a small grid.  The march above walks zc + 2 planes one after the
+// other and each is a round trip to memory; where a launch has few cells that chain is
+// its whole time.  Here a workgroup owns a bx x by x bz block of output cells and holds
+// step one of the block and its one-cell halo in LDS, one cell per lane: one round trip,
+// step one, one barrier, step two, for 2 - 3 times the step-one work of the march.
+// Channel + sphere, fp32 BGK / MRT per launch, march before and now: (24, 24, 48) 10.6 ->
+// 5.5 / 13.1 -> 6.5 us, 48^3 12.7 -> 8.7 / 16.5 -> 10.1 us, 60^3 13.7 -> 13.2 / 17.2 ->
+// 14.9 us.  Its workgroups are numbered like the march's tiles: neighbouring blocks share
+// an XCD's L2, without which the halos are fetched up to eight times (60^3: 24 us).
+//
+// `div` holds ceil(2^20 / d) for the divisors of the lane and block numbers, all below
+// 1024: n / d = n * div >> 20.
+constexpr int kBlockCells = 1024;
+
+struct Block2 {
+  int bx, by, bz;
+  uint32_t div_ex, div_ey, div_bx, div_by, div_ntx, div_nty;
+};
+
+template <class L, int S, int COLL, int FEAT, int BCK>
+__global__ __launch_bounds__(kBlockCells) void k_lbm2_block(const KArgs<typename Store<S>::C> a, const Block2 b) {
+  using T = typename Store<S>::T;
+  using C = typename Store<S>::C;
+  constexpr int Q = L::Q;
+  constexpr bool kAll = (FEAT & FEAT_BC) != 0;
+  constexpr bool kDevIn = dev_in<S, COLL, FEAT>();
+  static_assert((FEAT & (FEAT_MLP | FEAT_FORCE)) == 0, "plain steps only");
+  __shared__ T s[Q * kBlockCells];
+  __shared__ uint8_t s_solid[kAll ? kBlockCells : 1];
+  __shared__ C s_eq[kAll ? Q : 1];
+  const int t = threadIdx.x;
+  const int nx = a.nx, ny = a.ny, nz = a.nz;
+  const int EX = b.bx + 2, EY = b.by + 2, EZ = b.bz + 2;
+  const auto div = [](int n, uint32_t m) { return int((uint32_t(n) * m) >> 20); };
+  const auto wrap = [](int c, int n) { return c < 0 ? c + n : (c >= n ? c - n : c); };
+  const int tile = int(xcd_tile(blockIdx.x, gridDim.x));
+  const int ntx = (nx + b.bx - 1) / b.bx, nty = (ny + b.by - 1) / b.by;
+  const int row = div(tile, b.div_ntx), iz = div(row, b.div_nty);
+  const int x0 = (tile - row * ntx) * b.bx, y0 = (row - iz * nty) * b.by, z0 = iz * b.bz;
+  const T* fin = static_cast<const T*>(a.fin);
+  // step-one cell of this lane; a block is no larger than the grid, so its halo wraps at most once
+  const bool h1 = t < EX * EY * EZ;
+  const int r1 = h1 ? div(t, b.div_ex) : 0, lx = h1 ? t - r1 * EX : 0, lz = div(r1, b.div_ey), ly = r1 - lz * EY;
+  const int gx = wrap(x0 - 1 + lx, nx), gy = wrap(y0 - 1 + ly, ny), gz = wrap(z0 - 1 + lz, nz);
+  bool nb_edge = false;
+  if constexpr (kAll) {
+    const int bck = BCK == BCK_RUNTIME ? a.bc_kind : BCK;
+    nb_edge = (bck == TLBM_BC_CHANNEL_X && (gx == 0 || gx == nx - 1)) ||
+              (bck == TLBM_BC_FAR_FIELD && gx == nx - 1 && !(a.bc_faces & TLBM_FACE_XP_PERIODIC));
+  }
+  const int gxn = nb_edge ? (gx == 0 ? 1 : nx - 2) : gx;
+  double unused_force = 0.0;
+  C f[Q];
+  int mask = 0;
+  {
+    const int xd = wrap_dn(gxn, nx), xu = wrap_up(gxn, nx), yd = wrap_dn(gy, ny), yu = wrap_up(gy, ny);
+    const int zd = wrap_dn(gz, nz), zu = wrap_up(gz, nz);
+    if (h1) {
+      if constexpr (kAll) {
+        if (a.solid != nullptr) mask = a.solid[(uint32_t(gz) * uint32_t(ny) + uint32_t(gy)) * uint32_t(nx) + uint32_t(gx)];
+      }
+      // z differs from lane to lane here, so the offsets are 64-bit ones
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int64_t off = int64_t(src_of(L::cz[q], zd, gz, zu)) * a.isz +
+                            int64_t(src_of(L::cy[q], yd, gy, yu)) * a.isy + src_of(L::cx[q], xd, gxn, xu);
+        f[q] = take<L, S, kDevIn>(*(global_ptr<const T>)(fin + int64_t(q) * a.isq + off), q);
+      }
+    }
+  }
+  if constexpr (kAll) {
+    if (t == 0) {
+      C e[Q];
+      equilibrium_here<L>(C(1), a.bc_u, e);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) s_eq[q] = e[q];
+    }
+    lds_barrier();
+  }
+  auto eq_unit = [&](C (&e)[Q]) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) e[q] = s_eq[q];
+  };
+  if (h1) {
+    auto none = [](int, int, int, int) { return C(0); };
+    const uint32_t cell = (uint32_t(gz) * uint32_t(ny) + uint32_t(gy)) * uint32_t(nx) + uint32_t(gx);
+    update_cell<L, S, COLL, true, FEAT, BCN_IN_F, BCK, kDevIn>(f, a, gx, gy, gz, cell, mask != 0, nb_edge,
+                                                               unused_force, unused_force, unused_force, none, eq_unit);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) s[q * kBlockCells + t] = put_out<L, S, COLL, FEAT>(f[q], q);
+    if constexpr (kAll) s_solid[t] = mask != 0 ? 1 : 0;
+  }
+  lds_barrier();
+  // output cell of this lane; lanes past the grid redo its last cell and store nothing
+  const int n2 = b.bx * b.by * b.bz;
+  if (__builtin_amdgcn_readfirstlane(t) >= n2) return;
+  const int t2 = t < n2 ? t : 0;
+  const int r2 = div(t2, b.div_bx), tx = t2 - r2 * b.bx, tz = div(r2, b.div_by), ty = r2 - tz * b.by;
+  const bool own = t < n2 && x0 + tx < nx && y0 + ty < ny && z0 + tz < nz;
+  const int x = min(x0 + tx, nx - 1), y = min(y0 + ty, ny - 1), z = min(z0 + tz, nz - 1);
+  const int at = ((z - z0 + 1) * EY + (y - y0 + 1)) * EX + (x - x0 + 1);
+  const int plane = EX * EY;
+  auto lds_at = [&](int q, int px, int, int) -> C {
+    return take<L, S, kDevIn>(s[q * kBlockCells + at + (px - x) - L::cx[q] - L::cy[q] * EX - L::cz[q] * plane], q);
+  };
+#pragma unroll
+  for (int q = 0; q < Q; ++q) f[q] = lds_at(q, x, y, z);
+  bool solid = false;
+  if constexpr (kAll) solid = s_solid[at] != 0;
+  const uint32_t cell = (uint32_t(z) * uint32_t(ny) + uint32_t(y)) * uint32_t(nx) + uint32_t(x);
+  update_cell<L, S, COLL, true, FEAT, BCN_PULL, BCK, kDevIn>(f, a, x, y, z, cell, solid, false, unused_force,
+                                                             unused_force, unused_force, lds_at, eq_unit);
+  if (own) {
+    T* fout = static_cast<T*>(a.fout) + (int64_t(z) * a.osz + int64_t(y) * a.osy + x);
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      *(global_ptr<T>)(fout + int64_t(q) * a.osq) = put_out<L, S, COLL, FEAT>(f[q], q);
+  }
 }
 
 // The learned-closure step.  Its collision is long (the network runs on the
@@ -1911,6 +2032,79 @@ inline Plan2 plan2(int ny, int nx, int nz, int64_t pitch, int esize, int cells, 
   return s;
 }
 
+// Blocks of the small-grid kernel, or false where the march is to be taken: above 800
+// cells per compute unit.  Measured on 20 grids of 4 000 - 200 000 cells with five kernels
+// each, block against march: 1.8 - 2.0x up to 33 000 cells, 1.0 - 1.5x (mean 1.22x) at
+// 110 000 - 200 000; at 64^3, 1024 cells per unit, 0.85x.
+// Among the blocks that cut each axis into equal parts it takes the one with the least
+// rounds * (waves of both steps + cache lines of the pulled rows / 4); over those
+// launches it is within 2 % of the fastest block on average.
+inline bool block2(int ny, int nx, int nz, bool outlet, int cus, Block2* out) {
+  if (int64_t(nx) * ny > 800 * int64_t(cus) || int64_t(nx) * ny * nz > 800 * int64_t(cus)) return false;
+  if (outlet && nx < 4) return false;
+  // the distinct ceil(n / parts) of an axis, largest first, up to what the lanes can hold
+  const auto next = [](int n, int b) {  // the next smaller one, 0 after 1
+    if (b <= 1) return 0;
+    const int parts = (n + b - 2) / (b - 1);
+    return (n + parts - 1) / parts;
+  };
+  constexpr int widest = kBlockCells / 9 - 2;
+  const auto first = [](int n) { return n <= widest ? n : (n + (n + widest - 1) / widest - 1) / ((n + widest - 1) / widest); };
+  int best = INT_MAX;
+  for (int bx = first(nx); bx > 0; bx = next(nx, bx)) {
+    if (outlet && (nx - 1) % bx < 2) continue;  // as step2_reason for the march's tile
+    const int ntx = (nx + bx - 1) / bx;
+    for (int by = first(ny); by > 0; by = next(ny, by)) {
+      if ((bx + 2) * (by + 2) * 3 > kBlockCells) continue;
+      const int cols = ntx * ((ny + by - 1) / by);
+      if (cols >= 1024) break;
+      for (int bz = first(nz); bz > 0; bz = next(nz, bz)) {
+        const int cells = (bx + 2) * (by + 2) * (bz + 2);
+        if (cells > kBlockCells) continue;
+        const int w = cols * ((nz + bz - 1) / bz);
+        if (w >= 1024) break;
+        const int waves = (cells + 63) / 64 + (bx * by * bz + 63) / 64;
+        const int cost = (w + cus - 1) / cus * (128 * waves + (by + 2) * (bz + 2) * (bx + 34));
+        if (cost < best) {
+          best = cost;
+          out->bx = bx;
+          out->by = by;
+          out->bz = bz;
+        }
+      }
+    }
+  }
+  if (best == INT_MAX) return false;
+  const auto div = [](int d) { return uint32_t(((1 << 20) + d - 1) / d); };
+  out->div_ex = div(out->bx + 2);
+  out->div_ey = div(out->by + 2);
+  out->div_bx = div(out->bx);
+  out->div_by = div(out->by);
+  out->div_ntx = div((nx + out->bx - 1) / out->bx);
+  out->div_nty = div((ny + out->by - 1) / out->by);
+  return true;
+}
+
+// The search takes microseconds, as long as the launch it is for: each thread keeps the
+// result for the sizes it asked for last.
+inline const Block2* block2_of(int ny, int nx, int nz, bool outlet, int cus) {
+  struct Last {
+    int ny = 0, nx = 0, nz = 0, cus = 0;
+    bool outlet = false, found = false;
+    Block2 b{};
+  };
+  static thread_local Last l;
+  if (l.ny != ny || l.nx != nx || l.nz != nz || l.cus != cus || l.outlet != outlet) {
+    l.found = block2(ny, nx, nz, outlet, cus, &l.b);
+    l.ny = ny;
+    l.nx = nx;
+    l.nz = nz;
+    l.cus = cus;
+    l.outlet = outlet;
+  }
+  return l.found ? &l.b : nullptr;
+}
+
 // Batched lid-driven cavities, two steps per launch: the two-step march over the
 // column tiles of every cavity in one grid.  Cavity i (edge E, [z][q][y][x] at
 // element `offset` with the (y, x) plane padded to a multiple of 64) owns
@@ -2068,6 +2262,14 @@ int launch_lbm2(const KArgs<typename Store<S>::C>& a, hipStream_t s) {
   Plan2 p{width, 8, 1, 1};
   if constexpr (L::Q == 19) {
     const bool outlet = a.bc_kind == TLBM_BC_CHANNEL_X || a.bc_kind == TLBM_BC_FAR_FIELD;
+    if constexpr ((FEAT & FEAT_FORCE) == 0) {
+      if (const Block2* b = block2_of(a.ny, a.nx, a.nz, outlet, device_cus())) {
+        const int n = (a.nx + b->bx - 1) / b->bx * ((a.ny + b->by - 1) / b->by) * ((a.nz + b->bz - 1) / b->bz);
+        const int lanes = ((b->bx + 2) * (b->by + 2) * (b->bz + 2) + 63) / 64 * 64;
+        hipLaunchKernelGGL((k_lbm2_block<L, S, COLL, FEAT, BCK>), dim3(n), dim3(lanes), 0, s, a, *b);
+        return check_launch("k_lbm2_block");
+      }
+    }
     p = plan2(a.ny, a.nx, a.nz, a.osy, esize, cells, outlet, device_cus());
   } else {
     const int64_t cols = int64_t((a.nx + width - 1) / width) * ((a.ny + 7) / 8);
