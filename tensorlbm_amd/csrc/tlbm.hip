@@ -71,6 +71,7 @@ struct KArgs {
   int64_t osq, osz, osy;  // output strides
   int nx, ny, nz, tiles_x, tiles_y;
   int tau_mode, eq_floor, bc_kind, bc_faces;
+  int nt, rev, run;  // one-step kernels: kind of store and order of the tiles (set_sweep)
   uint32_t row_mul, row_shift;  // flat tiles: c / nx = umulhi(c, row_mul) >> row_shift; row_mul 0: tiles of rows
   C omega, tau, cs_delta_sq, tau_cap;
   C rate[8];
@@ -89,6 +90,13 @@ using global_ptr = __attribute__((address_space(1))) T*;
 template <typename T>
 __device__ __forceinline__ T ld_off(const T* base, uint32_t off) {
   return *(global_ptr<const T>)(reinterpret_cast<const char*>(base) + off * uint32_t(sizeof(T)));
+}
+
+// the same, not kept in the caches: for values that nothing reads again
+template <typename T>
+__device__ __forceinline__ T ld_nt(const T* base, uint32_t off) {
+  return __builtin_nontemporal_load(
+      (global_ptr<const T>)(reinterpret_cast<const char*>(base) + off * uint32_t(sizeof(T))));
 }
 
 // A pointer the caller knows to be uniform over the wave, moved to scalar registers
@@ -502,6 +510,35 @@ __device__ __forceinline__ void force_flush(double* force, double fx, double fy,
   }
 }
 
+// Workgroup w of a 1-D grid of n runs on XCD w % 8 (round-robin dispatch over the
+// 8 dies, each with its own L2).  Give XCD c the contiguous tile range c*n/8 ..
+// so that tiles sharing halo rows (x and y neighbours, x fastest) run at the same
+// time on the same die and meet their halo lines in that die's L2.
+constexpr uint32_t kXcds = 8;
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t w, uint32_t n) {
+  const uint32_t q = n / kXcds, r = n % kXcds;  // XCDs below r take q + 1 tiles
+  const uint32_t c = w % kXcds, slot = w / kXcds;
+  return c < r ? c * (q + 1) + slot : r * (q + 1) + (c - r) * q + slot;
+}
+
+// The order of the elementwise ops and of one-step kernels with ordinary stores on rows
+// of partial lines: runs of 16 workgroups per XCD (`run`).  With consecutive
+// workgroups on different XCDs an XCD only ever touches every eighth block of 256 cells.  Where the populations lie a power
+// of two apart (128^3) these all fall on the same half or quarter of its L2's channels: fp64
+// 128^3 collide 131 -> 115 us, macroscopic 75 -> 67 us; runs of 4 / 64 117 - 133 us, a whole
+// eighth of the grid per XCD the same there and 5 % slower at 128 x 128 x 192.  And a line
+// that two blocks share is fetched by two L2s, or written by both: fused fp16 step of
+// 200 x 200 x 250 188 -> 157 us.  Rows of whole lines share none, and the fused step, whose
+// lattices are padded apart, loses there (fp32 256^3 421 -> 434 us).
+// `rev`: last workgroup first.
+constexpr uint32_t kRun = 16;
+__device__ __forceinline__ uint32_t sweep_tile(uint32_t w, uint32_t n, bool rev, bool run) {
+  if (rev) w = n - 1 - w;
+  if (!run || w >= n / (kXcds * kRun) * (kXcds * kRun)) return w;
+  const uint32_t c = w % kXcds, k = w / kXcds;
+  return (k / kRun * kXcds + c) * kRun + k % kRun;
+}
+
 // Whether the lane at x takes, before the update, the pulled state of the cell
 // its boundary reads (x = 1 for the channel inlet, x = nx - 2 for a copy outlet),
 // so that `pulled` can hand back its own f: only lanes whose boundary reads it.
@@ -521,7 +558,7 @@ constexpr bool flat_tiles() {
   return (FEAT & FEAT_MLP) == 0 && (!STREAM || (FEAT & FEAT_BC) == 0 || (FEAT & FEAT_FORCE) != 0);
 }
 
-template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK>
+template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK, bool NT>
 __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
   using ST = Store<S>;
   using T = typename ST::T;
@@ -530,7 +567,9 @@ __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
   constexpr bool kAll = (FEAT & FEAT_BC) != 0;
   constexpr bool kDevIn = dev_in<S, COLL, FEAT>();
 
-  const uint32_t tile = blockIdx.x;
+  // the orders go with ordinary stores (set_sweep), but for the ops
+  constexpr bool kSweep = !NT || COLL == TLBM_COLL_NONE;
+  const uint32_t tile = kSweep ? sweep_tile(blockIdx.x, gridDim.x, a.rev != 0, a.run != 0) : blockIdx.x;
   int x, y, z;
   bool active;
   if (flat_tiles<STREAM, FEAT>() && a.row_mul != 0) {
@@ -562,7 +601,7 @@ __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
   } else {
     const uint32_t off = uint32_t(yy) * uint32_t(a.isy) + uint32_t(xx);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) f[q] = ST::template get<L>(ld_off(fin + int64_t(q) * a.isq + int64_t(z) * a.isz, off), q);
+    for (int q = 0; q < Q; ++q) f[q] = ST::template get<L>(ld_nt(fin + int64_t(q) * a.isq + int64_t(z) * a.isz, off), q);
   }
   // (issued after the gather: measured faster here than ahead of it, unlike the
   // two-step kernel's prefetch)
@@ -599,22 +638,15 @@ __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
     T* fout = static_cast<T*>(a.fout);
     const uint32_t off = uint32_t(yy) * uint32_t(a.osy) + uint32_t(xx);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, put_out<L, S, COLL, FEAT>(f[q], q));
+    for (int q = 0; q < Q; ++q) {
+      T* base = fout + int64_t(q) * a.osq + int64_t(z) * a.osz;
+      if constexpr (NT) st_nt(base, off, put_out<L, S, COLL, FEAT>(f[q], q));
+      else st_l2(base, off, put_out<L, S, COLL, FEAT>(f[q], q));
+    }
   }
   if constexpr ((FEAT & FEAT_FORCE) != 0) {
     if (a.force != nullptr) force_flush(a.force, fx, fy, fz, solid);
   }
-}
-
-// Workgroup w of a 1-D grid of n runs on XCD w % 8 (round-robin dispatch over the
-// 8 dies, each with its own L2).  Give XCD c the contiguous tile range c*n/8 ..
-// so that tiles sharing halo rows (x and y neighbours, x fastest) run at the same
-// time on the same die and meet their halo lines in that die's L2.
-constexpr uint32_t kXcds = 8;
-__device__ __forceinline__ uint32_t xcd_tile(uint32_t w, uint32_t n) {
-  const uint32_t q = n / kXcds, r = n % kXcds;  // XCDs below r take q + 1 tiles
-  const uint32_t c = w % kXcds, slot = w / kXcds;
-  return c < r ? c * (q + 1) + slot : r * (q + 1) + (c - r) * q + slot;
 }
 
 // Vector-memory counter of gfx9-family parts: it counts loads and stores, in
@@ -914,9 +946,9 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
   }
 }
 
-template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK>
+template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK, bool NT>
 __global__ __launch_bounds__(256) void k_lbm(const KArgs<typename Store<S>::C> a) {
-  lbm_body<L, S, COLL, STREAM, FEAT, BCK>(a);
+  lbm_body<L, S, COLL, STREAM, FEAT, BCK, NT>(a);
 }
 
 template <class L, int S, int COLL, int FEAT, int BCK>
@@ -1246,7 +1278,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TLBM_MLP_WA
     lbm_mlp_body<L, S, COLL, STREAM, FEAT, BCK>(a, zper);
   } else {
     (void)zper;
-    lbm_body<L, S, COLL, STREAM, FEAT, BCK>(a);
+    lbm_body<L, S, COLL, STREAM, FEAT, BCK, true>(a);
   }
 }
 
@@ -1265,9 +1297,12 @@ __global__ __launch_bounds__(256) void k_equilibrium(const T* rho, const T* ux, 
   for (int q = 0; q < L::Q; ++q) out[uint64_t(q) * N + i] = feq[q];
 }
 
+// `rev`: the last cells first, which of a large lattice are the ones still in the
+// memory-side cache (128^3 fp64 after a boundary op:
+// 92 -> 67 us)
 template <class L, typename T>
-__global__ __launch_bounds__(256) void k_macroscopic(const T* f, T* rho, T* ux, T* uy, T* uz, uint64_t N) {
-  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_macroscopic(const T* f, T* rho, T* ux, T* uy, T* uz, uint64_t N, int rev) {
+  const uint64_t i = uint64_t(sweep_tile(blockIdx.x, gridDim.x, rev != 0, true)) * blockDim.x + threadIdx.x;
   if (i >= N) return;
   T v[L::Q];
 #pragma unroll
@@ -1306,14 +1341,14 @@ __global__ __launch_bounds__(256) void k_boundary(const T* fin, T* fout, int nz,
   using L = D3Q19;
   constexpr int Q = L::Q;
   const uint64_t N = uint64_t(nz) * ny * nx;
-  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const uint64_t i = uint64_t(sweep_tile(blockIdx.x, gridDim.x, false, true)) * blockDim.x + threadIdx.x;
   if (i >= N) return;
-  const int x = int(i % uint64_t(nx));
-  const int y = int((i / uint64_t(nx)) % uint64_t(ny));
-  const int z = int(i / (uint64_t(nx) * ny));
+  const uint32_t r = uint32_t(i) / uint32_t(nx);  // N < 2^31
+  const int x = int(uint32_t(i) - r * uint32_t(nx));
+  const int z = int(r / uint32_t(ny)), y = int(r) - z * ny;
   T f[Q];
 #pragma unroll
-  for (int q = 0; q < Q; ++q) f[q] = fin[uint64_t(q) * N + i];
+  for (int q = 0; q < Q; ++q) f[q] = __builtin_nontemporal_load(fin + uint64_t(q) * N + i);
   if (kind == TLBM_BC_CHANNEL_X) {
     if (x == 0) {  // equilibrium inlet, u = (u_in, 0, 0), density of x = 1
       T rho1 = T(0);
@@ -1864,6 +1899,31 @@ int fill_args(KArgs<C>& a, int lattice, const void* fin, const int64_t* is, void
 
 // ---- instantiation table ----------------------------------------------------
 
+// One-step kernels built with ordinary stores beside the non-temporal ones: the stream op,
+// the fused BGK step, the 16-bit and obstacle forms that have no two-step kernel or do not
+// use it, and the unit-rate cumulants.  A choice at run time would keep the conversions and
+// stores of the first populations from starting before the others' collision is done
+// (unit-rate cumulants 256^3 fp16: 308 -> 343 us per step).
+template <class L, int S, int COLL, bool STREAM, int FEAT>
+constexpr bool both_stores() {
+  if (!STREAM || (FEAT & FEAT_MLP) != 0) return false;
+  if (COLL == TLBM_COLL_NONE || COLL == COLL_GEIER_UNIT) return true;
+  if (L::Q != 19 || S == ST_F16 || S == ST_BF16) return false;
+  return COLL == TLBM_COLL_BGK || (FEAT & FEAT_FORCE) != 0;
+}
+
+template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK>
+int launch_k_lbm(const KArgs<typename Store<S>::C>& a, dim3 grid, dim3 block, hipStream_t s) {
+  if constexpr (both_stores<L, S, COLL, STREAM, FEAT>()) {
+    if (!a.nt) {
+      hipLaunchKernelGGL((k_lbm<L, S, COLL, STREAM, FEAT, BCK, false>), grid, block, 0, s, a);
+      return check_launch("k_lbm");
+    }
+  }
+  hipLaunchKernelGGL((k_lbm<L, S, COLL, STREAM, FEAT, BCK, STREAM>), grid, block, 0, s, a);
+  return check_launch("k_lbm");
+}
+
 template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK = BCK_RUNTIME>
 int launch_lbm(const KArgs<typename Store<S>::C>& a, int bx, int by, uint32_t nb, hipStream_t s) {
   if constexpr ((FEAT & FEAT_MLP) != 0) {
@@ -1888,12 +1948,10 @@ int launch_lbm(const KArgs<typename Store<S>::C>& a, int bx, int by, uint32_t nb
         b.row_shift = uint32_t(k - 1);
         b.tiles_x = int((uint64_t(a.nx) * uint64_t(a.ny) + 255) / 256);
         b.tiles_y = 1;
-        hipLaunchKernelGGL((k_lbm<L, S, COLL, STREAM, FEAT, BCK>), dim3(uint32_t(b.tiles_x) * uint32_t(a.nz)),
-                           dim3(256), 0, s, b);
-        return check_launch("k_lbm");
+        return launch_k_lbm<L, S, COLL, STREAM, FEAT, BCK>(b, dim3(uint32_t(b.tiles_x) * uint32_t(a.nz)), dim3(256), s);
       }
     }
-    hipLaunchKernelGGL((k_lbm<L, S, COLL, STREAM, FEAT, BCK>), dim3(nb), dim3(bx, by), 0, s, a);
+    return launch_k_lbm<L, S, COLL, STREAM, FEAT, BCK>(a, dim3(nb), dim3(bx, by), s);
   }
   return check_launch("k_lbm");
 }
@@ -2327,7 +2385,47 @@ struct Call {
   const tlbm_boundary* bc;
   double* force;
   hipStream_t s;
+  bool rev;
 };
+
+// From this lattice size on two of them no longer share the 256 MB memory-side cache.
+constexpr double kSweepMB = 145.0;
+
+// How a one-step launch uses that cache, which keeps what went through it last: ordinary
+// loads and stores enter it, non-temporal ones do not.
+//
+// Stores (a.nt).  Up to kSweepMB the next launch finds what this one wrote; above, keeping
+// this one's input there for the launch after is worth more.  Rows that end in the middle of
+// a 32-byte sector go through L2, where their two halves meet: above 256 MB only where they
+// miss 16 bytes as well.  Below 20 MB the L2s serve either way.  fp32 / fp16 D3Q19 channel
+// and D3Q27, non-temporal against ordinary, us per step: 55 MB 25.2 / 20.4, 75 MB 33.6 /
+// 27.6, 137 MB 51.2 / 50.5, 174 MB 62.1 / 64.4, 221 MB 78.0 / 83.0, 638 MB 214 / 219; rows
+// of 300 bytes, 128 MB, 73.0 / 65.1; of 500, 380 MB, 223 / 188; of 272, 234 MB, 101 / 104
+// (99 / 86 in the two orders below); of 400, 432 MB, 148 / 156.
+//
+// Order.  Above kSweepMB a launch that starts where the one before it stopped finds the end
+// of that one's output in the cache, if it was put there: every second step of a run (a.rev;
+// 160 x 180 x 193 fp32 182 -> 175 us, 200 x 200 x 250 fp16 157 -> 152), and the collide op,
+// which follows a boundary or stream op.  A tile of a small lattice should rather meet the L2
+// of the XCD that wrote it (64^3 fp16 6.8 us, reversed 8.4).  a.run: see sweep_tile.
+//
+// A collide op's input and output: read past the caches, written into them; a stream op's
+// output, which one more op reads, the other way round above kSweepMB.
+template <class L, int S, int COLL, typename C>
+void set_sweep(KArgs<C>& a, bool streams, bool rev) {
+  constexpr int esize = int(sizeof(typename Store<S>::T));
+  const double mb = 1e-6 * L::Q * esize * double(a.nz) * a.ny * a.nx;
+  const int64_t row = (a.osy | a.nx) * esize;
+  const bool op = COLL == TLBM_COLL_NONE;
+  if (mb < 20.0) {
+    a.nt = !op;
+  } else {
+    a.nt = row % 32 == 0 ? mb > kSweepMB : (row % 16 == 0 && mb > 256.0);
+  }
+  if (!streams) a.nt = 0;
+  a.rev = (rev || !streams) && !a.nt && mb > kSweepMB;
+  a.run = op || !streams || (!a.nt && row % 128 != 0);
+}
 
 template <class L, int S, int COLL>
 int run_coll(const Call& c) {
@@ -2340,6 +2438,7 @@ int run_coll(const Call& c) {
     int rc = fill_args(a, c.lattice, c.fin, c.is, c.fout, c.os, c.nz, c.ny, c.nx, c.coll, c.solid, c.bc, c.force, &bx,
                        &by, &nb);
     if (rc != TLBM_OK) return rc;
+    set_sweep<L, S, COLL>(a, c.stream_, c.rev);
     if (c.coll != nullptr && c.coll->tau_mode == TLBM_TAU_MLP) {
       if constexpr (L::Q == 19 && COLL == TLBM_COLL_BGK) {
         if (!c.stream_) return fail(TLBM_ERR_UNSUPPORTED, "the learned closure runs in the fused step");
@@ -2553,9 +2652,9 @@ const char* tlbm_status_string(int status) {
   }
 }
 
-int tlbm_step(int lattice, int store, const void* f_in, const int64_t* in_strides, void* f_out,
+static int step_one_launch(int lattice, int store, const void* f_in, const int64_t* in_strides, void* f_out,
               const int64_t* out_strides, int nz, int ny, int nx, const tlbm_collision* coll, const int8_t* solid,
-              const tlbm_boundary* bc, double* force, tlbm_stream_t stream) {
+              const tlbm_boundary* bc, double* force, bool rev, tlbm_stream_t stream) {
   g_err[0] = 0;
   int64_t is[3], os[3];
   int rc = prepare(lattice, store, f_in, in_strides, f_out, out_strides, nz, ny, nx, is, os);
@@ -2567,8 +2666,15 @@ int tlbm_step(int lattice, int store, const void* f_in, const int64_t* in_stride
   const bool feat = solid != nullptr || force != nullptr || (bc != nullptr && bc->kind != TLBM_BC_NONE);
   if (force != nullptr && solid == nullptr) return fail(TLBM_ERR_INVALID, "force needs a solid mask");
   Call c{lattice, store, coll->kind, true, feat, 1, f_in, is, f_out, os, nz, ny, nx, coll, solid, bc, force,
-         (hipStream_t)stream};
+         (hipStream_t)stream, rev};
   return run(c);
+}
+
+int tlbm_step(int lattice, int store, const void* f_in, const int64_t* in_strides, void* f_out,
+              const int64_t* out_strides, int nz, int ny, int nx, const tlbm_collision* coll, const int8_t* solid,
+              const tlbm_boundary* bc, double* force, tlbm_stream_t stream) {
+  return step_one_launch(lattice, store, f_in, in_strides, f_out, out_strides, nz, ny, nx, coll, solid, bc, force, false,
+                         stream);
 }
 
 int tlbm_step2(int lattice, int store, const void* f_in, const int64_t* in_strides, void* f_out,
@@ -2586,7 +2692,7 @@ int tlbm_step2(int lattice, int store, const void* f_in, const int64_t* in_strid
     return fail(TLBM_ERR_UNSUPPORTED, "the two-step force sample is built for D3Q19; sample D3Q27 with tlbm_step");
   const bool feat = solid != nullptr || force != nullptr || (bc != nullptr && bc->kind != TLBM_BC_NONE);
   Call c{lattice, store, coll->kind, true, feat, 2, f_in, is, f_out, os, nz, ny, nx, coll, solid, bc, force,
-         (hipStream_t)stream};
+         (hipStream_t)stream, false};
   return run(c);
 }
 
@@ -2605,7 +2711,8 @@ int tlbm_run(int lattice, int store, const void* f_in, const int64_t* in_strides
     void* out = to ? buf_b : buf_a;
     const bool two = pairs && n_steps - k >= 2;
     const int rc = two ? tlbm_step2(lattice, store, in, is, out, buf_strides, nz, ny, nx, coll, solid, bc, nullptr, stream)
-                       : tlbm_step(lattice, store, in, is, out, buf_strides, nz, ny, nx, coll, solid, bc, nullptr, stream);
+                       : step_one_launch(lattice, store, in, is, out, buf_strides, nz, ny, nx, coll, solid, bc, nullptr,
+                                         k % 2 == 1, stream);
     if (rc != TLBM_OK) return rc;
     *last = to;
     in = out;
@@ -2627,7 +2734,7 @@ int tlbm_stream(int lattice, int store, const void* f_in, const int64_t* in_stri
   if (rc) return rc;
   if (f_in == f_out) return fail(TLBM_ERR_ALIAS, "f_in and f_out alias; streaming needs two buffers");
   Call c{lattice, store, TLBM_COLL_NONE, true, false, 1, f_in, is, f_out, os, nz, ny, nx, nullptr, nullptr, nullptr,
-         nullptr, (hipStream_t)stream};
+         nullptr, (hipStream_t)stream, false};
   return run(c);
 }
 
@@ -2642,7 +2749,7 @@ int tlbm_collide(int lattice, int store, const void* f_in, const int64_t* in_str
   if (rc) return rc;
   if (coll == nullptr || coll->kind == TLBM_COLL_NONE) return fail(TLBM_ERR_INVALID, "collision kind required");
   Call c{lattice, store, coll->kind, false, false, 1, f_in, is, f_out, os, nz, ny, nx, coll, nullptr, nullptr, nullptr,
-         (hipStream_t)stream};
+         (hipStream_t)stream, false};
   return run(c);
 }
 
@@ -2682,10 +2789,10 @@ int tlbm_macroscopic(int lattice, int dtype, const void* f, void* rho, void* ux,
     using L = decltype(lat);
     if (dtype == TLBM_STORE_F32) {
       hipLaunchKernelGGL((k_macroscopic<L, float>), dim3(blocks_for(n)), dim3(256), 0, s, (const float*)f,
-                         (float*)rho, (float*)ux, (float*)uy, (float*)uz, n);
+                         (float*)rho, (float*)ux, (float*)uy, (float*)uz, n, int(4e-6 * L::Q * n > kSweepMB));
     } else if (dtype == TLBM_STORE_F64) {
       hipLaunchKernelGGL((k_macroscopic<L, double>), dim3(blocks_for(n)), dim3(256), 0, s, (const double*)f,
-                         (double*)rho, (double*)ux, (double*)uy, (double*)uz, n);
+                         (double*)rho, (double*)ux, (double*)uy, (double*)uz, n, int(8e-6 * L::Q * n > kSweepMB));
     } else {
       return fail(TLBM_ERR_DTYPE, "macroscopic takes float32 or float64 populations");
     }
