@@ -522,14 +522,14 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t w, uint32_t n) {
 }
 
 // The order of the elementwise ops and of one-step kernels with ordinary stores on rows
-// of partial lines: runs of 16 workgroups per XCD (`run`).  With consecutive
-// workgroups on different XCDs an XCD only ever touches every eighth block of 256 cells.  Where the populations lie a power
-// of two apart (128^3) these all fall on the same half or quarter of its L2's channels: fp64
-// 128^3 collide 131 -> 115 us, macroscopic 75 -> 67 us; runs of 4 / 64 117 - 133 us, a whole
-// eighth of the grid per XCD the same there and 5 % slower at 128 x 128 x 192.  And a line
-// that two blocks share is fetched by two L2s, or written by both: fused fp16 step of
-// 200 x 200 x 250 188 -> 157 us.  Rows of whole lines share none, and the fused step, whose
-// lattices are padded apart, loses there (fp32 256^3 421 -> 434 us).
+// of partial lines: runs of 16 workgroups per XCD (`run`).  With consecutive workgroups on
+// different XCDs an XCD only ever touches every eighth block of 256 cells.  Where the
+// populations lie a power of two apart (128^3) these all fall on the same half or quarter of
+// its L2's channels: fp64 128^3 collide 131 -> 115 us, macroscopic 75 -> 67 us; runs of 4 /
+// 64 117 - 133 us, a whole eighth of the grid per XCD the same there and 5 % slower at
+// 128 x 128 x 192.  And a line that two blocks share is fetched by two L2s, or written by
+// both: fused fp16 step of 200 x 200 x 250 188 -> 157 us.  Rows of whole lines share none,
+// and the fused step, whose lattices are padded apart, loses there (fp32 256^3 421 -> 434 us).
 // `rev`: last workgroup first.
 constexpr uint32_t kRun = 16;
 __device__ __forceinline__ uint32_t sweep_tile(uint32_t w, uint32_t n, bool rev, bool run) {
@@ -1085,7 +1085,7 @@ __global__ __launch_bounds__(kBlockCells) void k_lbm2_block(const KArgs<typename
 // solid byte) are loaded while the current plane is collided, and the network's
 // operand blob is staged once into LDS, whose reads count on the LDS counter
 // and so never wait behind the prefetch as global reads of the blob would.
-template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK>
+template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK, bool NT>
 __device__ __forceinline__ void lbm_mlp_body(const KArgs<typename Store<S>::C>& a, int zper) {
   static_assert(STREAM, "the learned closure runs in the fused step");
   using ST = Store<S>;
@@ -1237,8 +1237,11 @@ __device__ __forceinline__ void lbm_mlp_body(const KArgs<typename Store<S>::C>& 
     uint32_t offl = off;
     asm volatile("" : "+v"(offl));
 #pragma unroll
-    for (int q = 0; q < Q; ++q)
-      st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, offl, put_out<L, S, COLL, FEAT>(f[q], q));
+    for (int q = 0; q < Q; ++q) {
+      T* base = fout + int64_t(q) * a.osq + int64_t(z) * a.osz;
+      if constexpr (NT) st_nt(base, offl, put_out<L, S, COLL, FEAT>(f[q], q));
+      else st_l2(base, offl, put_out<L, S, COLL, FEAT>(f[q], q));
+    }
   }
   if constexpr ((FEAT & FEAT_FORCE) != 0) {
     if (a.force != nullptr)
@@ -1271,14 +1274,14 @@ constexpr bool mlp_marches() {
   return S == ST_F16 || S == ST_BF16 || S == ST_F16_DEV || S == ST_BF16_DEV;
 }
 
-template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK>
+template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK, bool NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TLBM_MLP_WAVES))) void k_lbm_mlp(
     const KArgs<typename Store<S>::C> a, int zper) {
   if constexpr (mlp_marches<S>()) {
-    lbm_mlp_body<L, S, COLL, STREAM, FEAT, BCK>(a, zper);
+    lbm_mlp_body<L, S, COLL, STREAM, FEAT, BCK, NT>(a, zper);
   } else {
     (void)zper;
-    lbm_body<L, S, COLL, STREAM, FEAT, BCK, true>(a);
+    lbm_body<L, S, COLL, STREAM, FEAT, BCK, NT>(a);
   }
 }
 
@@ -1927,12 +1930,28 @@ int launch_k_lbm(const KArgs<typename Store<S>::C>& a, dim3 grid, dim3 block, hi
 template <class L, int S, int COLL, bool STREAM, int FEAT, int BCK = BCK_RUNTIME>
 int launch_lbm(const KArgs<typename Store<S>::C>& a, int bx, int by, uint32_t nb, hipStream_t s) {
   if constexpr ((FEAT & FEAT_MLP) != 0) {
-    // nb = tiles_x * tiles_y * nz; the closure step marches zper planes per workgroup
-    const uint32_t cols = uint32_t(a.tiles_x) * uint32_t(a.tiles_y);
+    // The closure step marches zper planes per workgroup.  Its 4- and 8-byte form runs lanes
+    // past the row's end through the network with the rest, so its tiles are 64 wide where
+    // wider ones leave whole waves of them (160^3 fp32 143 -> 125 us, 100^3 38 -> 32 us).
+    KArgs<typename Store<S>::C> b = a;
+    if (!mlp_marches<S>() && a.tiles_x * bx > (a.nx + 63) / 64 * 64) {
+      bx = 64;
+      by = 4;
+      b.tiles_x = (a.nx + 63) / 64;
+      b.tiles_y = (a.ny + 3) / 4;
+    }
+    const uint32_t cols = uint32_t(b.tiles_x) * uint32_t(b.tiles_y);
     const int zper = mlp_marches<S>() ? mlp_zper(cols, a.nz) : 1;
-    const uint32_t nbz = cols * uint32_t((a.nz + zper - 1) / zper);
+    const uint64_t nbz = uint64_t(cols) * uint64_t((a.nz + zper - 1) / zper);
     (void)nb;
-    hipLaunchKernelGGL((k_lbm_mlp<L, S, COLL, STREAM, FEAT, BCK>), dim3(nbz), dim3(bx, by), 0, s, a, zper);
+    if (nbz >= (uint64_t(1) << 31)) return fail(TLBM_ERR_SHAPE, "too many workgroups");
+    // stores as set_sweep says: fp16 150 x 160 x 190 123 -> 107 us per step, 180 x 190 x 135 151 -> 131
+    if (a.nt)
+      hipLaunchKernelGGL((k_lbm_mlp<L, S, COLL, STREAM, FEAT, BCK, true>), dim3(uint32_t(nbz)), dim3(bx, by), 0, s, b,
+                         zper);
+    else
+      hipLaunchKernelGGL((k_lbm_mlp<L, S, COLL, STREAM, FEAT, BCK, false>), dim3(uint32_t(nbz)), dim3(bx, by), 0, s, b,
+                         zper);
   } else {
     // Rows that do not fill their waves: tiles of consecutive cells, y and x by one
     // multiply.  96 x 96 x 193 with force and LES: four waves a row, the fourth with one

@@ -90,6 +90,25 @@ def test_repeated_obstacles(collision, nx, copies):
         assert bool(((total / k - force).abs() <= 1e-9 * force.abs().max()).all())
 
 
+# rows of 140, 280 and 384 bytes; tiles of 64 x 4 (70, 150) and of whole rows (96)
+@pytest.mark.parametrize("dtype,boundary,nx,copies", [
+    (torch.float16, "channel_x", 70, (15, 90)), (torch.bfloat16, None, 150, (6, 45)),
+    (torch.float32, "channel_x", 70, (8, 50)), (torch.float32, None, 150, (4, 30)), (torch.float32, "lid_y", 96, (6, 30)),
+])
+def test_repeated_closures(dtype, boundary, nx, copies):
+    shape = (10, 67, nx)
+    f, solid = _state(19, shape, dtype), _solid(shape)
+    kw = dict(deviation=dtype != torch.float32, boundary=boundary, u_bc=(0.04, 0.0, 0.0), C_s=0.17,
+              closure=tl.EddyViscosityMLP3D("cuda:0", seed=4))
+    ref = tl.FusedSolver3D(*shape, 0.55, "cuda:0", dtype, solid=solid if boundary else None, **kw).run(f, 3)[0].clone()
+    for k in copies:
+        big = tl.FusedSolver3D(shape[0] * k, *shape[1:], 0.55, "cuda:0", dtype,
+                               solid=solid.repeat(k, 1, 1) if boundary else None, **kw)
+        g = big.run(f.repeat(1, k, 1, 1), 3)[0]
+        for i in (0, k // 2, k - 1):
+            _same(ref, g[:, 10 * i:10 * (i + 1)])
+
+
 @pytest.mark.parametrize("dtype,shape", [(torch.float64, (101, 100, 102)), (torch.float32, (130, 128, 128)),
                                          (torch.float32, (31, 33, 35))])
 def test_ops_on_halves(dtype, shape):
