@@ -121,7 +121,7 @@ __global__ __launch_bounds__(CAV_TILE) void k_cavities(const CavArgs a) {
 
 // Every cavity at rest: one workgroup per (cavity, z, q) plane in turn, each plane one
 // value.  As 64 strided copies of an expanded vector this took 3.6 ms for 64 cavities of
-// edges 32-160; as one launch 1.0 ms.
+// edges 32-160; as one launch 1.1 ms.
 template <int S>
 __global__ __launch_bounds__(256) void k_cav_fill(const CavArgs a, uint32_t planes) {
   using T = typename Store<S>::T;
