@@ -1305,7 +1305,7 @@ __global__ __launch_bounds__(256) void k_equilibrium(const T* rho, const T* ux, 
 
 // `rev`: the last cells first, which of a large lattice are the ones still in the
 // memory-side cache (128^3 fp64 after a boundary op:
-// 92 -> 67 us)
+// 92 -> 74 us)
 template <class L, typename T>
 __global__ __launch_bounds__(256) void k_macroscopic(const T* f, T* rho, T* ux, T* uy, T* uz, uint64_t N, int rev) {
   const uint64_t i = uint64_t(sweep_tile(blockIdx.x, gridDim.x, rev != 0, true)) * blockDim.x + threadIdx.x;
