@@ -13,6 +13,9 @@ import os
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 LIB_NAME = "libtlbm_hip.so"
 LIB_PATH = Path(__file__).with_name(LIB_NAME)
@@ -236,6 +239,31 @@ def stream_of(t: torch.Tensor) -> int:
     if _raw_stream is not None:
         return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def on_current_device(t: torch.Tensor) -> bool:
+    """Whether launches on torch's current stream of the tensor's device reach that device."""
+    return t.get_device() == torch.cuda.current_device()
+
+
+def eager_write(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may read and write these tensors by address in place of torch's in-place operators:
+    plain tensors on the current device, with no gradient, tangent or transform (vmap, grad, functionalize) on
+    them and no dispatch or function mode, tracer or compiler watching; inference tensors only in inference mode."""
+    if torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() or \
+            torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
+    if torch._C._len_torch_function_stack() and not all(
+            isinstance(m, DeviceContext) for m in _get_current_function_mode_stack()):
+        return False
+    for t in tensors:
+        if type(t) is not torch.Tensor or t.requires_grad or t.is_neg() or not on_current_device(t):
+            return False
+        if t.is_inference() and not torch.is_inference_mode_enabled():
+            return False
+        if forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None:
+            return False
+    return True
 
 
 def require_gpu(t: torch.Tensor, what: str) -> None:

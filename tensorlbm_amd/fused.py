@@ -219,18 +219,13 @@ def fused_obstacle_step(
     if force is None and acc is not None:
         dt = fx_buf.dtype
         if dt in (torch.float32, torch.float64) and all(
-                b.numel() == 1 and b.dtype == dt and b.device == f.device and _plain(b) for b in bufs):
+                b.numel() == 1 and b.dtype == dt and b.device == f.device for b in bufs) and nat.eager_write(*bufs):
             nat.check(nat.lib().tlbm_force_add(nat.store_code(dt), acc.data_ptr(), *(b.data_ptr() for b in bufs),
                                                nat.stream_of(f)), "fused_obstacle_step")
         else:
             for i, b in enumerate(bufs):
                 b.add_(acc[i].to(b.dtype))
     return out
-
-
-def _plain(t: torch.Tensor) -> bool:
-    """A tensor that a kernel may write in place without torch seeing it: no subclass, no autograd."""
-    return type(t) is torch.Tensor and not t.requires_grad
 
 
 def _distinct(f: torch.Tensor) -> bool:
@@ -255,14 +250,15 @@ def apply_far_field_bc_6face(f: torch.Tensor, u_in: float, *, uy: float = 0.0, u
     ``f`` holds absolute populations, shape ``(Q, nz, ny, nx)`` with Q ≥ 19 (slots past 19 are set to 0,
     as the reference pads its 32-slot buffers).  ``feq_vec`` (shape ``(19,)`` or ``(Q,)``) skips the
     equilibrium.  One launch writes every face (``tlbm_far_field_faces``; a plane copy each where ``f`` is
-    no plain dense floating-point tensor); ``FusedSolver3D(boundary="far_field")`` applies the same faces
-    inside the step instead.
+    no dense floating-point tensor or more than an eager write is asked for: tangents, vmap, tracing);
+    ``FusedSolver3D(boundary="far_field")`` applies the same faces inside the step instead.
     """
     if f.dim() != 4 or f.shape[0] < 19:
         raise ValueError(f"f must be (Q >= 19, nz, ny, nx), got shape {tuple(f.shape)}")
     nat.require_gpu(f, "apply_far_field_bc_6face")
     q, nz, ny, nx = (int(v) for v in f.shape)
-    launch = f.dtype in (torch.float32, torch.float64, torch.float16, torch.bfloat16) and _plain(f) and _distinct(f)
+    launch = f.dtype in (torch.float32, torch.float64, torch.float16, torch.bfloat16) and _distinct(f) and \
+        nat.eager_write(f)
     if launch and feq_vec is None and q == 19 and f.dtype in (torch.float32, torch.float64):
         u = (ctypes.c_double * 3)(float(u_in), float(uy), float(uz))
         nat.check(nat.lib().tlbm_far_field_faces(nat.store_code(f.dtype), q, f.data_ptr(), nat.strides_of(f), nz, ny,
@@ -286,7 +282,7 @@ def apply_far_field_bc_6face(f: torch.Tensor, u_in: float, *, uy: float = 0.0, u
         feq_vec = feq_pad_buf
     elif feq_vec.shape[0] > q:
         feq_vec = feq_vec[:q]
-    if launch and _plain(feq_vec):
+    if launch and nat.eager_write(feq_vec):
         feq_vec = feq_vec.contiguous()
         nat.check(nat.lib().tlbm_far_field_faces(nat.store_code(f.dtype), q, f.data_ptr(), nat.strides_of(f), nz, ny,
                                                  nx, None, feq_vec.data_ptr(), nat.stream_of(f)),
