@@ -266,6 +266,14 @@ def eager_write(*tensors: torch.Tensor) -> bool:
     return True
 
 
+def written(*tensors: torch.Tensor) -> None:
+    """Tell autograd of a kernel's write, as an in-place operator does, so that a backward pass that saved one of
+    these tensors raises instead of using the new values."""
+    for t in tensors:
+        if not t.is_inference():
+            torch.autograd.graph.increment_version(t)
+
+
 def require_gpu(t: torch.Tensor, what: str) -> None:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{what} must be a torch.Tensor")

@@ -222,6 +222,7 @@ def fused_obstacle_step(
                 b.numel() == 1 and b.dtype == dt and b.device == f.device for b in bufs) and nat.eager_write(*bufs):
             nat.check(nat.lib().tlbm_force_add(nat.store_code(dt), acc.data_ptr(), *(b.data_ptr() for b in bufs),
                                                nat.stream_of(f)), "fused_obstacle_step")
+            nat.written(*bufs)
         else:
             for i, b in enumerate(bufs):
                 b.add_(acc[i].to(b.dtype))
@@ -263,6 +264,7 @@ def apply_far_field_bc_6face(f: torch.Tensor, u_in: float, *, uy: float = 0.0, u
         u = (ctypes.c_double * 3)(float(u_in), float(uy), float(uz))
         nat.check(nat.lib().tlbm_far_field_faces(nat.store_code(f.dtype), q, f.data_ptr(), nat.strides_of(f), nz, ny,
                                                  nx, u, None, nat.stream_of(f)), "apply_far_field_bc_6face")
+        nat.written(f)
         return
     if feq_vec is None:
         from .ops import equilibrium3d
@@ -287,6 +289,7 @@ def apply_far_field_bc_6face(f: torch.Tensor, u_in: float, *, uy: float = 0.0, u
         nat.check(nat.lib().tlbm_far_field_faces(nat.store_code(f.dtype), q, f.data_ptr(), nat.strides_of(f), nz, ny,
                                                  nx, None, feq_vec.data_ptr(), nat.stream_of(f)),
                   "apply_far_field_bc_6face")
+        nat.written(f)
         return
     face = feq_vec[:, None, None]
     f[:, :, :, 0] = face

@@ -145,3 +145,31 @@ def test_force_buffers_carry_tangents(where):
             d = fw.unpack_dual(b)
             assert float(d.primal) == 2.0 * i + 1.0 and float(d.tangent) == 0.5 + i
     assert not calls
+
+
+def test_saved_tensors_notice_the_launch(where):
+    device, calls = where
+    f, feq = _state(device), _state(device, 1)[:, 0, 0, 0].contiguous()
+    w = torch.ones((), device=device, requires_grad=True)
+    for given in ({"feq_vec": feq}, {}):  # both forms of the launch
+        loss = (w * f).sum()
+        tl.apply_far_field_bc_6face(f[:, :, :, :], 0.05, **given)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            loss.backward()
+    bufs = [torch.ones(1, device=device) for _ in range(3)]
+    loss = sum((w * b).sum() for b in bufs)
+    versions = [b._version for b in bufs]
+    _force(f, bufs, None)
+    assert [b._version for b in bufs] == [v + 1 for v in versions]
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
+    assert calls is None or calls == ["tlbm_far_field_faces", "tlbm_far_field_faces", "tlbm_force_add"]
+
+
+def test_launches_in_inference_mode(where):
+    device, calls = where
+    with torch.inference_mode():
+        f = _state(device)
+        tl.apply_far_field_bc_6face(f, 0.05, feq_vec=f[:, 0, 0, 0].clone())
+        _force(f, [f[i, 0, 0, :1].clone() for i in range(3)], None)
+    assert calls is None or calls == ["tlbm_far_field_faces", "tlbm_force_add"]
