@@ -259,7 +259,7 @@ def apply_far_field_bc_6face(f: torch.Tensor, u_in: float, *, uy: float = 0.0, u
     nat.require_gpu(f, "apply_far_field_bc_6face")
     q, nz, ny, nx = (int(v) for v in f.shape)
     launch = f.dtype in (torch.float32, torch.float64, torch.float16, torch.bfloat16) and _distinct(f) and \
-        nat.eager_write(f)
+        q < 2**16 and nz * ny * nx < 2**31 and nat.eager_write(f)
     if launch and feq_vec is None and q == 19 and f.dtype in (torch.float32, torch.float64):
         u = (ctypes.c_double * 3)(float(u_in), float(uy), float(uz))
         nat.check(nat.lib().tlbm_far_field_faces(nat.store_code(f.dtype), q, f.data_ptr(), nat.strides_of(f), nz, ny,

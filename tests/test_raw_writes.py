@@ -173,3 +173,16 @@ def test_launches_in_inference_mode(where):
         tl.apply_far_field_bc_6face(f, 0.05, feq_vec=f[:, 0, 0, 0].clone())
         _force(f, [f[i, 0, 0, :1].clone() for i in range(3)], None)
     assert calls is None or calls == ["tlbm_far_field_faces", "tlbm_force_add"]
+
+
+@pytest.mark.parametrize("shape", [(19, 2, 2, 2**29), (65536, 2, 2, 3)])
+def test_faces_beyond_the_launch_limits(monkeypatch, shape):
+    """2^31 cells (82 GB in half precision) or 65536 populations: more than the launch takes, plane by plane then."""
+    lib = CountingLibrary()
+    monkeypatch.setattr(nat, "lib", lambda: lib)
+    monkeypatch.setattr(nat, "require_gpu", lambda t, what: None)
+    monkeypatch.setattr(nat, "stream_of", lambda t: 0)
+    monkeypatch.setattr(nat, "on_current_device", lambda t: True)
+    f = torch.empty(shape, dtype=torch.float16, device="meta")
+    tl.apply_far_field_bc_6face(f, 0.05, feq_vec=torch.empty(19, device="meta"))
+    assert not lib.calls
