@@ -120,11 +120,19 @@ def equilibrium27(rho, ux, uy, uz, device=None, *, out=None):
     return _equilibrium(27, rho, ux, uy, uz, out, "equilibrium27")
 
 
+def _new_like(f):
+    """Uninitialised plain contiguous tensor of f's shape, type and device (empty_like builds it in half the host
+    time, but hands on a subclass and the strides of axes of one cell)."""
+    if type(f) is torch.Tensor:
+        return torch.empty_like(f, memory_format=torch.contiguous_format)
+    return torch.empty(f.shape, dtype=f.dtype, device=f.device)
+
+
 def _macroscopic(f, q, what):
     f, dims = _pops(f, q, what)
     dt = _eager_dtype(f, what)
-    rho, ux, uy = (torch.empty_like(f[0]) for _ in range(3))
-    uz = torch.empty_like(f[0]) if q != 9 else None
+    rho, ux, uy = (_new_like(f[0]) for _ in range(3))
+    uz = _new_like(f[0]) if q != 9 else None
     rc = nat.lib().tlbm_macroscopic(q, dt, f.data_ptr(), rho.data_ptr(), ux.data_ptr(), uy.data_ptr(),
                                     nat.ptr(uz), dims[0] * dims[1] * dims[2], nat.stream_of(f))
     nat.check(rc, what)
@@ -443,7 +451,7 @@ def _stream(f, q, what):
     f, dims = _pops(f, q, what, contiguous=False)
     store = nat.store_code(f.dtype)
     dense = f.is_contiguous()
-    out = torch.empty_like(f) if dense else torch.empty(f.shape, dtype=f.dtype, device=f.device)
+    out = _new_like(f)
     rc = nat.lib().tlbm_stream(q, store, f.data_ptr(), None if dense else nat.strides_of(f), out.data_ptr(), None,
                                *dims, nat.stream_of(f))
     nat.check(rc, what)
