@@ -674,6 +674,7 @@ int tlbm_mlp_train_epoch(float* params, const float* x, const float* t, const in
 int tlbm_coarsen_moments(int lattice, int store, const void* f, const int64_t* strides, int nz, int ny, int nx,
                          int factor, float* out, tlbm_stream_t stream) {
   if (!f || !out) return cfail(TLBM_ERR_INVALID, "null pointer");
+  if (nz < 1 || ny < 1 || nx < 1) return cfail(TLBM_ERR_SHAPE, "grid dims must be >= 1");
   if (factor < 1 || nx % factor || ny % factor || nz % factor)
     return cfail(TLBM_ERR_SHAPE, "grid dims must be multiples of the coarsening factor");
   if (lattice != TLBM_D3Q19 && lattice != TLBM_D3Q27) return cfail(TLBM_ERR_UNSUPPORTED, "3-D lattices only");
