@@ -153,8 +153,9 @@ int cfail(int code, const char* fmt, long long v = 0) {
   return tlbm::set_error(code, buf);
 }
 
+// `steps`: the launch relaxes, so every tau must be stable (filling takes any)
 int build_args(CavArgs& a, int store, const void* f_in, void* f_out, const tlbm_cavity* cavs, int n,
-               int64_t capacity, double u_lid) {
+               int64_t capacity, double u_lid, bool steps = true) {
   if (!f_in || !f_out || !cavs) return cfail(TLBM_ERR_INVALID, "null pointer");
   if (f_in == f_out) return cfail(TLBM_ERR_ALIAS, "input and output alias");
   if (n < 1 || n > CAV_MAX) return cfail(TLBM_ERR_SHAPE, "cavity count must be 1..%lld", CAV_MAX);
@@ -170,7 +171,7 @@ int build_args(CavArgs& a, int store, const void* f_in, void* f_out, const tlbm_
   for (int i = 0; i < n; ++i) {
     const int E = cavs[i].edge;
     if (E < 3 || E > 1024) return cfail(TLBM_ERR_SHAPE, "cavity edge must be 3..1024 (got %lld)", E);
-    if (!(cavs[i].tau > 0.5)) return cfail(TLBM_ERR_INVALID, "cavity %lld: tau must be > 0.5", i);
+    if (steps && !(cavs[i].tau > 0.5)) return cfail(TLBM_ERR_INVALID, "cavity %lld: tau must be > 0.5", i);
     const int64_t size = int64_t(E) * 19 * cav_plane(E);
     if (cavs[i].offset < end || cavs[i].offset % 64 != 0)
       return cfail(TLBM_ERR_SHAPE, "cavity %lld: offsets must be 64-aligned, increasing and non-overlapping", i);
@@ -273,7 +274,7 @@ int tlbm_cavities_layout(tlbm_cavity* cavs, int n, int64_t* total_elements, int6
 int tlbm_cavities_fill(int store, void* f, int64_t capacity, const tlbm_cavity* cavs, int n, tlbm_stream_t stream) {
   CavArgs a;
   // (the table's check wants two buffers; only the second is used)
-  const int rc = build_args(a, store, static_cast<char*>(f) + 1, f, cavs, n, capacity, 0.0);
+  const int rc = build_args(a, store, static_cast<char*>(f) + 1, f, cavs, n, capacity, 0.0, false);
   if (rc != TLBM_OK) return rc;
   if (!f) return cfail(TLBM_ERR_INVALID, "null pointer");
   uint32_t planes = 0;

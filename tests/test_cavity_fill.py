@@ -1,0 +1,40 @@
+"""The state of rest of a cavity batch: what fill_equilibrium takes and how autograd hears of it."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+import tensorlbm_amd as tl
+from tensorlbm_amd import _native as nat
+
+
+@pytest.mark.parametrize("tau", [0.5, 0.3, 0.0, -1.0, float("nan")])
+def test_fill_does_not_ask_for_a_stable_tau(tau):
+    """The relaxation time has no part in the state of rest; the steps refuse it (host side, no GPU work)."""
+    table = (nat.Cavity * 1)()
+    table[0].edge, table[0].tau = 4, tau
+    n = ctypes.c_int64()
+    nat.check(nat.lib().tlbm_cavities_layout(table, 1, ctypes.byref(n), None), "layout")
+    a, b = ctypes.c_void_p(0x1000), ctypes.c_void_p(0x2000)
+    # (a capacity too small by one ends the call before a launch, after the other checks of the cavity)
+    args = (n.value - 1, table, 1)
+    assert nat.lib().tlbm_cavities_fill(nat.STORE_F32, a, *args, None) == nat.ERR_SHAPE
+    assert b"capacity" in nat.lib().tlbm_last_error()
+    assert nat.lib().tlbm_cavities_step(nat.STORE_F32, a, b, *args, 0.1, 0, None) == nat.ERR_INVALID
+    assert b"tau must be" in nat.lib().tlbm_last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,deviation", [(torch.float32, False), (torch.float16, True)])
+def test_fill_of_cavities_that_cannot_step(dtype, deviation):
+    c = tl.BatchedCavities([5, 9], [0.5, 0.7], dtype=dtype, deviation=deviation)
+    c.fill_equilibrium()
+    w = tl.lattice.D3Q19.W_EXACT64.to("cuda:0").reshape(19, 1, 1, 1)
+    for i in range(2):
+        want = (torch.zeros_like(w) if deviation else w).to(dtype).expand_as(c.cavity(i))
+        assert torch.equal(c.cavity(i), want)
+    with pytest.raises(ValueError, match="tau must be"):
+        c.step()
