@@ -108,16 +108,19 @@ class BatchedCavities:
 
     def fill_equilibrium(self) -> None:
         """ρ = 1, u = 0 everywhere (stored as f − w for deviation storage)."""
-        if self._store in (nat.STORE_F32, nat.STORE_F64, nat.STORE_F16_DEV, nat.STORE_BF16_DEV):
+        if self._store in (nat.STORE_F32, nat.STORE_F64, nat.STORE_F16_DEV, nat.STORE_BF16_DEV) and \
+                nat.eager_write(self.a):
             nat.check(nat.lib().tlbm_cavities_fill(self._store, self.a.data_ptr(), self.a.numel(), self._table,
                                                    self.n, nat.stream_of(self.a)), "tlbm_cavities_fill")
+            nat.written(self.a)
             return
-        from .lattice import D3Q19  # plain 16-bit storage, which no cavity step takes
+        # plain 16-bit storage, which no cavity step takes, and buffers that torch must see written
+        from .lattice import D3Q19
 
         w = D3Q19.W_EXACT64.to(self.device)
         for i in range(self.n):
             v = self.cavity(i)
-            v.copy_(w.reshape(19, 1, 1, 1).expand_as(v))
+            v.copy_((torch.zeros_like(w) if self.deviation else w).reshape(19, 1, 1, 1).expand_as(v))
 
     def populations(self, i: int) -> torch.Tensor:
         """Cavity i's populations f as a contiguous (19, L, L, L) tensor (w added back for deviation storage)."""

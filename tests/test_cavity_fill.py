@@ -38,3 +38,48 @@ def test_fill_of_cavities_that_cannot_step(dtype, deviation):
         assert torch.equal(c.cavity(i), want)
     with pytest.raises(ValueError, match="tau must be"):
         c.step()
+
+
+class NoLibrary:
+    def __getattr__(self, name):
+        return lambda *a: 0
+
+
+def _batch(device, monkeypatch):
+    if device != "cpu":
+        return tl.BatchedCavities([5], [0.7])
+    c = object.__new__(tl.BatchedCavities)
+    c._table = (nat.Cavity * 1)()
+    c._table[0].edge, c._table[0].tau = 5, 0.7
+    n = ctypes.c_int64()
+    nat.check(nat.lib().tlbm_cavities_layout(c._table, 1, ctypes.byref(n), None), "layout")
+    c.n, c.edges, c.device, c.dtype, c.deviation = 1, [5], torch.device("cpu"), torch.float32, False
+    c._store, c.a = nat.STORE_F32, torch.zeros(n.value)
+    monkeypatch.setattr(nat, "lib", lambda: NoLibrary())
+    monkeypatch.setattr(nat, "stream_of", lambda t: 0)
+    monkeypatch.setattr(nat, "on_current_device", lambda t: True)
+    return c
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda:0", marks=pytest.mark.gpu)])
+def test_fill_is_a_write_to_autograd(device, monkeypatch):
+    c = _batch(device, monkeypatch)
+    w = torch.ones((), device=device, requires_grad=True)
+    loss = (w * c.cavity(0)).sum()
+    c.fill_equilibrium()
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda:0", marks=pytest.mark.gpu)])
+def test_fill_under_a_tangent(device, monkeypatch):
+    """A buffer with a tangent loses it, as under the operator the fill stands for."""
+    import torch.autograd.forward_ad as fw
+
+    c = _batch(device, monkeypatch)
+    w = tl.lattice.D3Q19.W_EXACT64.to(device, torch.float32).reshape(19, 1, 1, 1)
+    with fw.dual_level():
+        c.a = fw.make_dual(c.a, torch.ones_like(c.a))
+        c.fill_equilibrium()
+        d = fw.unpack_dual(c.cavity(0))
+        assert torch.equal(d.primal, w.expand_as(d.primal)) and not d.tangent.any()
