@@ -284,9 +284,7 @@ def apply_far_field_bc_6face(f: torch.Tensor, u_in: float, *, uy: float = 0.0, u
         feq_vec = feq_pad_buf
     elif feq_vec.shape[0] > q:
         feq_vec = feq_vec[:q]
-    # (a feq_vec that lies in f changes as the planes are written)
-    if launch and nat.eager_write(feq_vec) and \
-            feq_vec.untyped_storage().data_ptr() != f.untyped_storage().data_ptr():
+    if launch and nat.eager_write(feq_vec):
         feq_vec = feq_vec.contiguous()
         nat.check(nat.lib().tlbm_far_field_faces(nat.store_code(f.dtype), q, f.data_ptr(), nat.strides_of(f), nz, ny,
                                                  nx, None, feq_vec.data_ptr(), nat.stream_of(f)),
