@@ -1252,18 +1252,21 @@ __device__ __forceinline__ void lbm_mlp_body(const KArgs<typename Store<S>::C>& 
 // Planes marched per workgroup by the learned-closure step, for `cols` column tiles of
 // nz planes.  A longer march hides more of the loads and stages the blob less often, but
 // 1024 workgroups fill the chip (four to a CU) and a few rounds of them are needed for
-// the last one not to idle it: 16 planes where that leaves two rounds, else the march that
-// leaves four.
-// 256^3: 16 (279 us; 305 marching 4).  Smaller grids marched 16 planes with most
-// CUs idle: fp16 deviations, 150 x 130 x 100 78 -> 53 us, 180 x 170 x 160 146 -> 124 us,
-// 90 x 60 x 60 39.7 -> 14.1 us, 65 x 50 x 40 80.7 -> 12.5 us.  192^3, 2.25 rounds of 16:
-// 9 planes took 1 % longer.
+// the last one not to idle it: 16 planes where that leaves four rounds, else the march that
+// leaves four, of at most 8 planes.
+// Smaller grids marched 16 planes with most CUs idle: fp16 deviations, 150 x 130 x 100
+// 78 -> 53 us, 180 x 170 x 160 146 -> 124 us, 90 x 60 x 60 39.7 -> 14.1 us, 65 x 50 x 40
+// 80.7 -> 12.5 us.  Between 8 and 16 planes for four rounds, 8 / 16 planes, us per step (medians
+// of 9, spread up to 7): 181 x 182 x 192 122.6 / 124.4, 192^3 135.8 / 135.2, 192 x 400 x 120
+// 265 / 298, 140 x 300 x 150 167 / 180, 200 x 210 x 250 234 / 253, 300 x 330 x 128 230 / 232,
+// 224^3 231 / 234, 250 x 250 x 200 377 / 427; 10 and 12 planes lie between.  Above, 256^3
+// 297 / 291 (305 marching 4), 270 x 270 x 256 326 / 322, 320 x 320 x 256 458 / 452.
 inline int mlp_zper(uint64_t cols, int nz) {
   const double x = double(cols) * nz / 4096.0;
   if (x < 0.25) return 1;
-  if (x >= 8.0) return 16;
+  if (x >= 16.0) return 16;
   const int z = int(x + 0.5);
-  return z < 2 ? 2 : z;
+  return z < 2 ? 2 : (z > 8 ? 8 : z);
 }
 
 // The march pays where the step is bound by instruction issue, i.e. with 16-bit
