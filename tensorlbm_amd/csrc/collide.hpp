@@ -874,7 +874,7 @@ __device__ __forceinline__ void geier27(C (&f)[27], C rho_eq, const Macro<C>& mc
 //   k_221 = -6 ux^2 uy^2 uz + s_xx k_021 + s_yy k_201 + 4 s_xy k_111 + 2 (s_xz k_120 + s_yz k_210),
 //   k_222 = the sum over the set partitions of {x, x, y, y, z, z}   (and permutations).
 // The 16-bit forms of the D3Q27 step are bound by instruction issue: 256^3 decaying
-// turbulence, fp16 deviations, 395 us per step by geier27, 308 us here (5.9 TB/s).
+// turbulence, fp16 deviations, 398 us per step by geier27, 311 us here (5.8 TB/s).
 // kDev: f holds the deviations f - w_q on entry and on return.  Density and stress are
 // then sums of deviations (d_xx = m_xx - (rho - 1) / 3 - rho ux^2), and the weights'
 // eight nonzero raw moments are taken off before the inverse sweeps.

@@ -525,9 +525,9 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t w, uint32_t n) {
 // of partial lines: runs of 16 workgroups per XCD (`run`).  With consecutive workgroups on
 // different XCDs an XCD only ever touches every eighth block of 256 cells.  Where the
 // populations lie a power of two apart (128^3) these all fall on the same half or quarter of
-// its L2's channels: fp64 128^3 collide 131 -> 115 us, macroscopic 75 -> 67 us; runs of 4 /
-// 64 117 - 133 us, a whole eighth of the grid per XCD the same there and 5 % slower at
-// 128 x 128 x 192.  And a line that two blocks share is fetched by two L2s, or written by
+// its L2's channels: fp64 128^3 collide 115 -> 101 us (131 -> 115 where it starts at the first
+// workgroup; there runs of 4 / 64 117 - 133 us, a whole eighth of the grid per XCD the same
+// and 5 % slower at 128 x 128 x 192).  And a line that two blocks share is fetched by two L2s, or written by
 // both: fused fp16 step of 200 x 200 x 250 188 -> 157 us.  Rows of whole lines share none,
 // and the fused step, whose lattices are padded apart, loses there (fp32 256^3 421 -> 434 us).
 // `rev`: last workgroup first.
@@ -962,10 +962,11 @@ __global__ __launch_bounds__((tile2_threads<L, S>())) void k_lbm2(const KArgs<ty
 // its whole time.  Here a workgroup owns a bx x by x bz block of output cells and holds
 // step one of the block and its one-cell halo in LDS, one cell per lane: one round trip,
 // step one, one barrier, step two, for 2 - 3 times the step-one work of the march.
-// Channel + sphere, fp32 BGK / MRT per launch, march before and now: (24, 24, 48) 10.6 ->
-// 5.5 / 13.1 -> 6.5 us, 48^3 12.7 -> 8.7 / 16.5 -> 10.1 us, 60^3 13.7 -> 13.2 / 17.2 ->
-// 14.9 us.  Its workgroups are numbered like the march's tiles: neighbouring blocks share
-// an XCD's L2, without which the halos are fetched up to eight times (60^3: 24 us).
+// Channel + sphere, fp32 BGK / MRT per launch, march and block: (24, 24, 48) 9.6 -> 5.7 /
+// 11.7 -> 6.6 us, 48^3 10.8 -> 9.0 / 13.3 -> 10.3 us, 58^3 14.4 -> 13.1 / 18.0 -> 14.8 us.
+// Its workgroups are numbered like the march's tiles: neighbouring blocks share an XCD's L2,
+// without which the halos are fetched up to eight times (60^3, just above the line below
+// which the blocks are taken: 24 us instead of 13).
 //
 // `div` holds ceil(2^20 / d) for the divisors of the lane and block numbers, all below
 // 1024: n / d = n * div >> 20.
@@ -1620,7 +1621,7 @@ __global__ __launch_bounds__(256) void k_scale(void* fv, Layout lay, const doubl
 // edges, so every cell is written once with the value the last of them leaves.  The
 // outlet reads x = nx-2, which no face of its row writes (nx = 2: the inlet's value).
 // One launch instead of a plane copy per face and the small operators that built the
-// face value: 96 x 96 x 193 fp32, about 25 launches -> one of 15 us.  Lanes enumerate a
+// face value: 96 x 96 x 193 fp32, about 25 launches -> one of 11.6 us.  Lanes enumerate a
 // population's face cells: first the (z, y) pairs of the x faces, whose two cells lie
 // next to each other in memory (x = nx-1 of a row, x = 0 of the next), then the rows
 // of the y faces and the z planes, contiguous.  blockIdx.y: population.
@@ -1669,7 +1670,7 @@ __global__ void k_force_add(const double* acc, T* bx, T* by, T* bz) {
 // MASS_PIECE values, four neighbouring ones to a lane and eight loads in flight; runs
 // start at any element, which global memory operations allow.  The per-cell forms (k_moment_sums: four
 // FP64 sums and two 64-bit divisions per cell; k_scale) took 58 and 44 us on
-// 96 x 96 x 193 fp32; these take 24 and 42 us.  The sum leaves one FP64 partial per
+// 96 x 96 x 193 fp32; these take 22 and 42 us.  The sum leaves one FP64 partial per
 // workgroup, added up in a fixed order by every workgroup of the scaling, so there is
 // no atomic, nothing to clear and the result does not vary from run to run.
 constexpr int MASS_PIECE = 256 * 4 * 8;
@@ -2078,11 +2079,15 @@ inline double tile2_cost(int tx, int ty, int ny, int nx, int nz, int esize, int 
 // average, 0.98x-1.6x; e.g. (245, 185, 68) 143 -> 106 us, MRT 185 -> 119 us;
 // (131, 147, 211) MRT 199 -> 172 us.
 //
-// Stores: non-temporal where rows or whole tiles are contiguous lines (through L2 they
-// took 3-11 % longer).  Otherwise a tile's rows end in partial lines that only merge
-// with the neighbouring tile's in L2: through L2 is up to 1.4x faster, except where
-// one lattice takes 120-256 MB.  There the input still sits in the 256 MB last-level
-// cache, stores through L2 push it out (0.8x), and narrower tiles lose as well.
+// Stores: non-temporal where rows (a pitch of whole lines) or whole tiles are contiguous
+// lines (through L2 they took 3-11 % longer).  Otherwise a tile's rows end in partial lines
+// that only merge with the neighbouring tile's in L2: through L2 is up to 1.4x faster, with
+// two exceptions.  Where one lattice takes 120-256 MB the input still sits in the 256 MB
+// last-level cache, stores through L2 push it out (0.8x), and narrower tiles lose as well.
+// Below 45 MB both lattices stay in that cache and the base tile's stores are better kept
+// out of L2: in 57 of those launches, of 10-45 MB, through L2 took 4 % less to 8 % more (mean
+// 2.7 % more), in the 36 fp32 ones of 45-120 MB 16 % less to 3 % more (mean 3.2 % less; 16-bit
+// ones within 3 %).
 inline Plan2 plan2(int ny, int nx, int nz, int64_t pitch, int esize, int cells, bool outlet, int cus) {
   const auto rows = [&](int tx) {
     int ty = cells / (tx + 2) - 2;

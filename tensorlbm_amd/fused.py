@@ -352,7 +352,7 @@ class FusedSolver3D:
     D3Q19 with fp32 storage, where it pays on MI355X (256³ channel + sphere,
     GLUPS one / two steps per launch: BGK 39.0 / 68.2, MRT 39.6 / 58.2, CM
     39.7 / 55.4, cumulant 39.1 / 59.1); with 16-bit storage (fp16 76.1 / 74.6)
-    and for D3Q27 (Geier at unit rates, fp16 54.5 / 52.3) the recomputed tile
+    and for D3Q27 (Geier at unit rates, fp16 54.3 / 52.3) the recomputed tile
     halo costs about what the saved traffic gains, or more.
     """
 
