@@ -707,6 +707,11 @@ template <class L, int S>
 constexpr int tile2_cells() {
   return 3 * L::Q * 66 * 10 * int(sizeof(typename Store<S>::T)) <= 158 * 1024 ? 66 * 10 : 34 * 10;
 }
+// width of the base tile, 8 rows high
+template <class L, int S>
+constexpr int tile2_width() {
+  return tile2_cells<L, S>() == 66 * 10 ? 64 : 32;
+}
 template <class L, int S>
 constexpr int tile2_threads() {
   return (tile2_cells<L, S>() + 63) / 64 * 64;
@@ -724,7 +729,11 @@ constexpr int tile2_threads() {
 // the solid cells are the five stationary walls of a cubic lid-driven cavity
 // (x = 0, x = nx-1, y = 0, z = 0, z = nz-1), decided from the coordinates
 // instead of read from a mask.
-template <class L, int S, int COLL, int FEAT, int BCK, bool BoxWalls = false>
+//
+// Tile: the output tile is a launch parameter (p2), or the base tile with non-temporal
+// stores, known at compile time.
+enum Tile2 { TILE_BASE, TILE_RUNTIME };
+template <class L, int S, int COLL, int FEAT, int BCK, Tile2 Tile, bool BoxWalls = false>
 __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, const Plan2& p2, uint32_t tile) {
   using ST = Store<S>;
   using T = typename ST::T;
@@ -732,11 +741,9 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
   constexpr int Q = L::Q;
   constexpr int EC = tile2_cells<L, S>();
   constexpr bool kDevIn = dev_in<S, COLL, FEAT>();
-  // The tile is a launch parameter: 64 x 8 where rows are whole cache lines, else the
-  // shape that wastes fewest lanes on this grid (plan2).  The LDS rows keep a fixed
-  // pitch of EC cells, so a run-time tile costs three more address registers than a
-  // compile-time one and nothing in the plane loop (256^3 channel: 480 us either way).
-  const int TX = p2.tx, TY = p2.ty, zc = p2.zc, EX = TX + 2;
+  // The LDS rows keep a fixed pitch of EC cells whatever the tile.
+  constexpr bool kBase = Tile == TILE_BASE;
+  const int TX = kBase ? tile2_width<L, S>() : p2.tx, TY = kBase ? 8 : p2.ty, zc = p2.zc, EX = TX + 2;
   constexpr bool kAll = (FEAT & FEAT_BC) != 0;
   constexpr bool kForce = (FEAT & FEAT_FORCE) != 0;
   static_assert((FEAT & FEAT_MLP) == 0, "the closure runs in the one-step kernel");
@@ -783,8 +790,9 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
   const bool h2 = t < TX * TY;
   const int ux_ = min(x0 + (h2 ? t % TX : 0), nx - 1), uy_ = min(y0 + (h2 ? t / TX : 0), ny - 1);
   const int ox = ux_ - x0, oy = uy_ - y0;
-  // tile cells of this lane's pulls by c_y (0, +1, -1), shifted by -c_x at the use
-  const int at_0 = (oy + 1) * EX + ox + 1, at_p = at_0 - EX, at_m = at_0 + EX;
+  // run-time tile: tile cells of this lane's pulls by c_y (0, +1, -1), shifted by -c_x at the
+  // use (a compile-time one forms them from the coordinates: held in registers they spill)
+  [[maybe_unused]] const int at_0 = (oy + 1) * EX + ox + 1, at_p = at_0 - EX, at_m = at_0 + EX;
   const bool own = h2 && x0 + t % TX < nx && y0 + t / TX < ny;
   double unused_force = 0.0;
   // Ladd force of both steps (obstacles.py:91-130), each cell of the launch's output range
@@ -893,17 +901,22 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
       // plane only: the boundary overrides read along x), written as plane
       // k + 1 - c_z[q] of the march
       const int row_a = set_row(-1, k + 2), row_b = set_row(0, k + 1), row_c = set_row(1, k);
-      auto lds_at = [&](int q, int x, int, int) -> C {  // only ever for this lane's y
+      auto lds_at = [&](int q, int x, int y, int) -> C {  // only ever for this lane's y
         const int row = (L::cz[q] < 0 ? row_a : L::cz[q] == 0 ? row_b : row_c) + R::index(q);
-        const int at = L::cy[q] == 0 ? at_0 : (L::cy[q] > 0 ? at_p : at_m);
-        return take<L, S, kDevIn>(s[row * EC + at + (x - ux_) - L::cx[q]], q);
+        if constexpr (kBase) {
+          const int sx = x - L::cx[q] - (x0 - 1), sy = y - L::cy[q] - (y0 - 1);
+          return take<L, S, kDevIn>(s[row * EC + sy * EX + sx], q);
+        } else {
+          const int at = L::cy[q] == 0 ? at_0 : (L::cy[q] > 0 ? at_p : at_m);
+          return take<L, S, kDevIn>(s[row * EC + at + (x - ux_) - L::cx[q]], q);
+        }
       };
       C f[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q) f[q] = lds_at(q, ux_, uy_, z);
       const uint32_t cell = (uint32_t(z) * uint32_t(ny) + uint32_t(uy_)) * uint32_t(nx) + uint32_t(ux_);
       bool solid = false;
-      if constexpr (kAll) solid = s_solid[((k + 1) % 3) * EC + at_0] != 0;
+      if constexpr (kAll) solid = s_solid[((k + 1) % 3) * EC + (oy + 1) * EX + (ox + 1)] != 0;
       if constexpr (kForce) {
         double sx = 0.0, sy = 0.0, sz = 0.0;
         update_cell<L, S, COLL, true, FEAT, BCN_PULL, BCK, kDevIn>(f, a, ux_, uy_, z, cell, solid, false, sx, sy, sz, lds_at,
@@ -920,21 +933,29 @@ __device__ __forceinline__ void lbm2_body(const KArgs<typename Store<S>::C>& a, 
       }
       T* fout = static_cast<T*>(a.fout);
       const uint32_t off = uint32_t(uy_) * uint32_t(a.osy) + uint32_t(ux_);
-      // Rounded before the choice of store: folded into the two store loops the last
-      // operations of the update would be contracted differently from the one-step kernel.
-      T o[Q];
+      if constexpr (kBase) {
+        if (own) {
 #pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        o[q] = put_out<L, S, COLL, FEAT>(f[q], q);
-        asm volatile("" : "+v"(o[q]));
-      }
-      if (own) {
-        if (p2.nt) {
+          for (int q = 0; q < Q; ++q)
+            st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, put_out<L, S, COLL, FEAT>(f[q], q));
+        }
+      } else {
+        // Rounded before the choice of store: folded into the two store loops the last
+        // operations of the update would be contracted differently from the one-step kernel.
+        T o[Q];
 #pragma unroll
-          for (int q = 0; q < Q; ++q) st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, o[q]);
-        } else {
+        for (int q = 0; q < Q; ++q) {
+          o[q] = put_out<L, S, COLL, FEAT>(f[q], q);
+          asm volatile("" : "+v"(o[q]));
+        }
+        if (own) {
+          if (p2.nt) {
 #pragma unroll
-          for (int q = 0; q < Q; ++q) st_l2(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, o[q]);
+            for (int q = 0; q < Q; ++q) st_nt(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, o[q]);
+          } else {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) st_l2(fout + int64_t(q) * a.osq + int64_t(z) * a.osz, off, o[q]);
+          }
         }
       }
     } else {
@@ -951,10 +972,16 @@ __global__ __launch_bounds__(256) void k_lbm(const KArgs<typename Store<S>::C> a
   lbm_body<L, S, COLL, STREAM, FEAT, BCK, NT>(a);
 }
 
-template <class L, int S, int COLL, int FEAT, int BCK>
+// The base tile's kernel is built with its shape at compile time beside the run-time form:
+// in the run-time form the index arithmetic of the pulls costs instructions and, with the
+// state of the force sample, registers.  Base tile, run-time / compile-time shape, us per
+// launch: fp32 MRT with force 256^3 767 / 595, 128^3 102 / 87; BGK with force 256^3 514 /
+// 485, without 482 / 464; fp16-deviation BGK channel 256^3 453 / 439; fp32 cumulant channel
+// 64^3 18.3 / 17.2; D3Q27 MRT 256^3 1074 / 1042.
+template <class L, int S, int COLL, int FEAT, int BCK, Tile2 Tile>
 __global__ __launch_bounds__((tile2_threads<L, S>())) void k_lbm2(const KArgs<typename Store<S>::C> a,
                                                                   const Plan2 p2) {
-  lbm2_body<L, S, COLL, FEAT, BCK>(a, p2, xcd_tile(blockIdx.x, gridDim.x));
+  lbm2_body<L, S, COLL, FEAT, BCK, Tile>(a, p2, xcd_tile(blockIdx.x, gridDim.x));
 }
 
 // Two fused steps of a small grid.  The march above walks zc + 2 planes one after the
@@ -2009,7 +2036,7 @@ int launch_lbm_kind(const KArgs<typename Store<S>::C>& a, int bx, int by, uint32
 // slower (518 against 480 us per launch): rows of 64 keep each pulled row in whole
 // cache lines.  Two half-size workgroups per CU (34 x 10 cells each, at most 128 VGPRs)
 // took 664-678 us.
-inline int tile2_width(int lattice, int store) {
+inline int tile2_width_of(int lattice, int store) {
   return lattice == TLBM_D3Q27 && store == TLBM_STORE_F32 ? 32 : 64;
 }
 
@@ -2245,7 +2272,7 @@ __global__ __launch_bounds__((tile2_threads<D3Q19, S>())) void k_cav2(
   k.omega = C(a.c[lo].omega);
   k.tau = C(1.0 / a.c[lo].omega);
   const Plan2 p2{a.c[lo].tx, a.c[lo].ty, a.zc, 0};
-  lbm2_body<D3Q19, S, TLBM_COLL_BGK, FEAT_BC, TLBM_BC_LID_Y, true>(k, p2, g - a.c[lo].tiles_before);
+  lbm2_body<D3Q19, S, TLBM_COLL_BGK, FEAT_BC, TLBM_BC_LID_Y, TILE_RUNTIME, true>(k, p2, g - a.c[lo].tiles_before);
 }
 
 // Output tile of a cavity of edge E: the base tile, the full row or the row in equal
@@ -2342,17 +2369,24 @@ inline const char* step2_reason(int lattice, int store, const tlbm_collision* co
   if (coll->tau_mode == TLBM_TAU_FIELD64) return "the fused step takes a float32 tau_eff field";
   if (bc != nullptr && (bc->kind == TLBM_BC_CHANNEL_X || bc->kind == TLBM_BC_FAR_FIELD)) {
     // the outlet copies x = nx-2, whose pulls reach x = nx-3: same tile as x = nx-1
-    if (nx < 4 || (nx - 1) % tile2_width(lattice, store) < 2) return "the outlet column would straddle two tiles";
+    if (nx < 4 || (nx - 1) % tile2_width_of(lattice, store) < 2) return "the outlet column would straddle two tiles";
   }
   return nullptr;
 }
 
+// Whether the two-step launch takes tiles by grid (plan2): D3Q19, and with a force sample BGK
+// only, whose boundary kind is known at compile time; the other force kernels lose more to
+// the run-time tile than it gains (fp32 MRT with force, 200 x 200 x 250 497 -> 573 us).
+template <class L, int COLL, int FEAT, int BCK>
+constexpr bool run_time_tile() {
+  return L::Q == 19 && ((FEAT & FEAT_FORCE) == 0 || (COLL == TLBM_COLL_BGK && BCK != BCK_RUNTIME));
+}
+
 template <class L, int S, int COLL, int FEAT, int BCK>
 int launch_lbm2(const KArgs<typename Store<S>::C>& a, hipStream_t s) {
-  constexpr int cells = tile2_cells<L, S>(), esize = sizeof(typename Store<S>::T);
-  constexpr int width = cells == 66 * 10 ? 64 : 32;
+  constexpr int cells = tile2_cells<L, S>(), esize = sizeof(typename Store<S>::T), width = tile2_width<L, S>();
   Plan2 p{width, 8, 1, 1};
-  if constexpr (L::Q == 19) {
+  if constexpr (run_time_tile<L, COLL, FEAT, BCK>()) {
     const bool outlet = a.bc_kind == TLBM_BC_CHANNEL_X || a.bc_kind == TLBM_BC_FAR_FIELD;
     if constexpr ((FEAT & FEAT_FORCE) == 0) {
       if (const Block2* b = block2_of(a.ny, a.nx, a.nz, outlet, device_cus())) {
@@ -2370,8 +2404,14 @@ int launch_lbm2(const KArgs<typename Store<S>::C>& a, hipStream_t s) {
   const uint64_t tiles = uint64_t((a.nx + p.tx - 1) / p.tx) * uint64_t((a.ny + p.ty - 1) / p.ty) *
                          uint64_t((a.nz + p.zc - 1) / p.zc);
   if (tiles >= (uint64_t(1) << 31)) return fail(TLBM_ERR_SHAPE, "too many workgroups");
-  hipLaunchKernelGGL((k_lbm2<L, S, COLL, FEAT, BCK>), dim3(uint32_t(tiles)), dim3(tile2_threads<L, S>()), 0, s, a,
-                     p);
+  const dim3 grid{uint32_t(tiles)}, block{uint32_t(tile2_threads<L, S>())};
+  if constexpr (run_time_tile<L, COLL, FEAT, BCK>()) {
+    if (p.tx != width || p.ty != 8 || !p.nt) {
+      hipLaunchKernelGGL((k_lbm2<L, S, COLL, FEAT, BCK, TILE_RUNTIME>), grid, block, 0, s, a, p);
+      return check_launch("k_lbm2");
+    }
+  }
+  hipLaunchKernelGGL((k_lbm2<L, S, COLL, FEAT, BCK, TILE_BASE>), grid, block, 0, s, a, p);
   return check_launch("k_lbm2");
 }
 
