@@ -601,7 +601,10 @@ __device__ __forceinline__ void lbm_body(const KArgs<typename Store<S>::C>& a) {
   } else {
     const uint32_t off = uint32_t(yy) * uint32_t(a.isy) + uint32_t(xx);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) f[q] = ST::template get<L>(ld_nt(fin + int64_t(q) * a.isq + int64_t(z) * a.isz, off), q);
+    for (int q = 0; q < Q; ++q) {
+      const T* base = fin + int64_t(q) * a.isq + int64_t(z) * a.isz;
+      f[q] = ST::template get<L>(NT ? ld_off(base, off) : ld_nt(base, off), q);
+    }
   }
   // (issued after the gather: measured faster here than ahead of it, unlike the
   // two-step kernel's prefetch)
@@ -1372,20 +1375,26 @@ __global__ __launch_bounds__(256) void k_bounce_back(const T* fin, T* fout, cons
 // read comes from the input, i.e. the state before any condition: the inlet's density from x = 1
 // and the outlet's copy of x = nx - 2 are taken before the lateral far-field faces are written, as
 // in boundaries3d.py:407-443 / 446-537 (nx >= 3 is checked on the host).
-template <typename T>
+// Cached: as the collide op above kOpsMB on rows of whole lines, ordinary loads and the plain
+// order (after collide and stream, fp64 256^3: far field 1002 against 949 us); else loads past
+// the caches and runs of workgroups per XCD (fp32 200^3 channel 280 -> 246 us).
+template <typename T, bool Cached>
 __global__ __launch_bounds__(256) void k_boundary(const T* fin, T* fout, int nz, int ny, int nx, int kind, int faces,
                                                   T bux, T buy, T buz, const int8_t* mask_a, const int8_t* mask_b) {
   using L = D3Q19;
   constexpr int Q = L::Q;
   const uint64_t N = uint64_t(nz) * ny * nx;
-  const uint64_t i = uint64_t(sweep_tile(blockIdx.x, gridDim.x, false, true)) * blockDim.x + threadIdx.x;
+  const uint64_t i = uint64_t(sweep_tile(blockIdx.x, gridDim.x, false, !Cached)) * blockDim.x + threadIdx.x;
   if (i >= N) return;
   const uint32_t r = uint32_t(i) / uint32_t(nx);  // N < 2^31
   const int x = int(uint32_t(i) - r * uint32_t(nx));
   const int z = int(r / uint32_t(ny)), y = int(r) - z * ny;
   T f[Q];
 #pragma unroll
-  for (int q = 0; q < Q; ++q) f[q] = __builtin_nontemporal_load(fin + uint64_t(q) * N + i);
+  for (int q = 0; q < Q; ++q) {
+    const T* at = fin + uint64_t(q) * N + i;
+    f[q] = Cached ? *at : __builtin_nontemporal_load(at);
+  }
   if (kind == TLBM_BC_CHANNEL_X) {
     if (x == 0) {  // equilibrium inlet, u = (u_in, 0, 0), density of x = 1
       T rho1 = T(0);
@@ -1936,14 +1945,15 @@ int fill_args(KArgs<C>& a, int lattice, const void* fin, const int64_t* is, void
 
 // ---- instantiation table ----------------------------------------------------
 
-// One-step kernels built with ordinary stores beside the non-temporal ones: the stream op,
-// the fused BGK step, the 16-bit and obstacle forms that have no two-step kernel or do not
+// One-step kernels built with ordinary stores beside the non-temporal ones: the stream and
+// collide ops, the fused BGK step, the 16-bit and obstacle forms that have no two-step kernel or do not
 // use it, and the unit-rate cumulants.  A choice at run time would keep the conversions and
 // stores of the first populations from starting before the others' collision is done
 // (unit-rate cumulants 256^3 fp16: 308 -> 343 us per step).
 template <class L, int S, int COLL, bool STREAM, int FEAT>
 constexpr bool both_stores() {
-  if (!STREAM || (FEAT & FEAT_MLP) != 0) return false;
+  if (!STREAM) return true;
+  if ((FEAT & FEAT_MLP) != 0) return false;
   if (COLL == TLBM_COLL_NONE || COLL == COLL_GEIER_UNIT) return true;
   if (L::Q != 19 || S == ST_F16 || S == ST_BF16) return false;
   return COLL == TLBM_COLL_BGK || (FEAT & FEAT_FORCE) != 0;
@@ -1957,7 +1967,7 @@ int launch_k_lbm(const KArgs<typename Store<S>::C>& a, dim3 grid, dim3 block, hi
       return check_launch("k_lbm");
     }
   }
-  hipLaunchKernelGGL((k_lbm<L, S, COLL, STREAM, FEAT, BCK, STREAM>), grid, block, 0, s, a);
+  hipLaunchKernelGGL((k_lbm<L, S, COLL, STREAM, FEAT, BCK, true>), grid, block, 0, s, a);
   return check_launch("k_lbm");
 }
 
@@ -2484,13 +2494,27 @@ constexpr double kSweepMB = 145.0;
 // of the XCD that wrote it (64^3 fp16 6.8 us, reversed 8.4).  a.run: see sweep_tile.
 //
 // A collide op's input and output: read past the caches, written into them; a stream op's
-// output, which one more op reads, the other way round above kSweepMB.
+// output, which one more op reads, the other way round above kSweepMB.  Above kOpsMB nothing
+// of one op's output is left for the next, and on rows of whole lines the ops do better with
+// non-temporal stores, ordinary loads and the plain order.  Caches and runs against that, us
+// for collide and for collide and stream in turn: fp32 256^3 474 and 1033 against 448 and 886,
+// D3Q27 fp32 128 x 128 x 256 (453 MB) 176 and 347 against 164 and 320, fp64 256^3 931 and 1870
+// against 896 and 1804, D2Q9 fp32 4096^2 212 and 433 against 203 and 403; at 319 MB 109 and 219
+// against 121 and 237.  Rows of partial lines keep them: fp32 200^3 233 and 448 against 311 and
+// 602.
+constexpr double kOpsMB = 330.0;
+
 template <class L, int S, int COLL, typename C>
 void set_sweep(KArgs<C>& a, bool streams, bool rev) {
   constexpr int esize = int(sizeof(typename Store<S>::T));
   const double mb = 1e-6 * L::Q * esize * double(a.nz) * a.ny * a.nx;
   const int64_t row = (a.osy | a.nx) * esize;
   const bool op = COLL == TLBM_COLL_NONE;
+  if ((op || !streams) && mb > kOpsMB && row % 128 == 0) {
+    a.nt = 1;
+    a.rev = a.run = 0;
+    return;
+  }
   if (mb < 20.0) {
     a.nt = !op;
   } else {
@@ -3093,16 +3117,16 @@ int tlbm_boundary_eager(int dtype, const void* f_in, void* f_out, int nz, int ny
   const double u0 = bc != nullptr ? bc->u[0] : 0.0, u1 = bc != nullptr ? bc->u[1] : 0.0,
                u2 = bc != nullptr ? bc->u[2] : 0.0;
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == TLBM_STORE_F32) {
-    hipLaunchKernelGGL(k_boundary<float>, dim3(blocks_for(n)), dim3(256), 0, s, (const float*)f_in, (float*)f_out, nz,
-                       ny, nx, kind, faces, float(u0), float(u1), float(u2), mask_a, mask_b);
-  } else if (dtype == TLBM_STORE_F64) {
-    hipLaunchKernelGGL(k_boundary<double>, dim3(blocks_for(n)), dim3(256), 0, s, (const double*)f_in,
-                       (double*)f_out, nz, ny, nx, kind, faces, u0, u1, u2, mask_a, mask_b);
-  } else {
-    return fail(TLBM_ERR_DTYPE, "boundary ops take float32 or float64 populations");
-  }
-  return check_launch("k_boundary");
+  const auto go = [&](auto t) -> int {
+    using T = decltype(t);
+    const bool cached = 19e-6 * sizeof(T) * double(n) > kOpsMB && nx * int64_t(sizeof(T)) % 128 == 0;
+    hipLaunchKernelGGL((cached ? k_boundary<T, true> : k_boundary<T, false>), dim3(blocks_for(n)), dim3(256), 0, s,
+                       (const T*)f_in, (T*)f_out, nz, ny, nx, kind, faces, T(u0), T(u1), T(u2), mask_a, mask_b);
+    return check_launch("k_boundary");
+  };
+  if (dtype == TLBM_STORE_F32) return go(float());
+  if (dtype == TLBM_STORE_F64) return go(double());
+  return fail(TLBM_ERR_DTYPE, "boundary ops take float32 or float64 populations");
 }
 
 int tlbm_sphere_mask(int nx, int ny, int nz, double cx, double cy, double cz, double radius, uint8_t* out,
