@@ -1337,12 +1337,14 @@ __global__ __launch_bounds__(256) void k_equilibrium(const T* rho, const T* ux, 
   for (int q = 0; q < L::Q; ++q) out[uint64_t(q) * N + i] = feq[q];
 }
 
-// `rev`: the last cells first, which of a large lattice are the ones still in the
-// memory-side cache (128^3 fp64 after a boundary op:
-// 92 -> 74 us)
+// `order` (macro_order): 1 runs of workgroups per XCD, 2 these from the last cells on, which of
+// a lattice somewhat larger than the memory-side cache are the ones still in it (128^3 fp64
+// after a boundary op: 92 -> 74 us); 0 as they come: with nothing left in the cache the runs
+// cost (fp32 256^3 290 against 272 us, D2Q9 fp32 6144^2 324 against 296).
 template <class L, typename T>
-__global__ __launch_bounds__(256) void k_macroscopic(const T* f, T* rho, T* ux, T* uy, T* uz, uint64_t N, int rev) {
-  const uint64_t i = uint64_t(sweep_tile(blockIdx.x, gridDim.x, rev != 0, true)) * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_macroscopic(const T* f, T* rho, T* ux, T* uy, T* uz, uint64_t N,
+                                                     int order) {
+  const uint64_t i = uint64_t(sweep_tile(blockIdx.x, gridDim.x, order == 2, order != 0)) * blockDim.x + threadIdx.x;
   if (i >= N) return;
   T v[L::Q];
 #pragma unroll
@@ -2504,6 +2506,8 @@ constexpr double kSweepMB = 145.0;
 // 602.
 constexpr double kOpsMB = 330.0;
 
+inline int macro_order(double mb) { return mb > kOpsMB ? 0 : (mb > kSweepMB ? 2 : 1); }
+
 template <class L, int S, int COLL, typename C>
 void set_sweep(KArgs<C>& a, bool streams, bool rev) {
   constexpr int esize = int(sizeof(typename Store<S>::T));
@@ -2887,10 +2891,10 @@ int tlbm_macroscopic(int lattice, int dtype, const void* f, void* rho, void* ux,
     using L = decltype(lat);
     if (dtype == TLBM_STORE_F32) {
       hipLaunchKernelGGL((k_macroscopic<L, float>), dim3(blocks_for(n)), dim3(256), 0, s, (const float*)f,
-                         (float*)rho, (float*)ux, (float*)uy, (float*)uz, n, int(4e-6 * L::Q * n > kSweepMB));
+                         (float*)rho, (float*)ux, (float*)uy, (float*)uz, n, macro_order(4e-6 * L::Q * n));
     } else if (dtype == TLBM_STORE_F64) {
       hipLaunchKernelGGL((k_macroscopic<L, double>), dim3(blocks_for(n)), dim3(256), 0, s, (const double*)f,
-                         (double*)rho, (double*)ux, (double*)uy, (double*)uz, n, int(8e-6 * L::Q * n > kSweepMB));
+                         (double*)rho, (double*)ux, (double*)uy, (double*)uz, n, macro_order(8e-6 * L::Q * n));
     } else {
       return fail(TLBM_ERR_DTYPE, "macroscopic takes float32 or float64 populations");
     }
