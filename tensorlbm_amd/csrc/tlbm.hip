@@ -1948,15 +1948,17 @@ int fill_args(KArgs<C>& a, int lattice, const void* fin, const int64_t* is, void
 // ---- instantiation table ----------------------------------------------------
 
 // One-step kernels built with ordinary stores beside the non-temporal ones: the stream and
-// collide ops, the fused BGK step, the 16-bit and obstacle forms that have no two-step kernel or do not
-// use it, and the unit-rate cumulants.  A choice at run time would keep the conversions and
-// stores of the first populations from starting before the others' collision is done
-// (unit-rate cumulants 256^3 fp16: 308 -> 343 us per step).
+// collide ops, the fused BGK step, the 16-bit and obstacle forms that have no two-step kernel
+// or do not use it, the D3Q27 steps with a mask or boundary and the unit-rate cumulants.  A
+// choice at run time would keep the conversions and stores of the first populations from
+// starting before the others' collision is done (unit-rate cumulants 256^3 fp16: 308 -> 343 us
+// per step).
 template <class L, int S, int COLL, bool STREAM, int FEAT>
 constexpr bool both_stores() {
   if (!STREAM) return true;
   if ((FEAT & FEAT_MLP) != 0) return false;
   if (COLL == TLBM_COLL_NONE || COLL == COLL_GEIER_UNIT) return true;
+  if (L::Q == 27) return FEAT != FEAT_NONE;
   if (L::Q != 19 || S == ST_F16 || S == ST_BF16) return false;
   return COLL == TLBM_COLL_BGK || (FEAT & FEAT_FORCE) != 0;
 }
@@ -2525,6 +2527,10 @@ void set_sweep(KArgs<C>& a, bool streams, bool rev) {
     a.nt = row % 32 == 0 ? mb > kSweepMB : (row % 16 == 0 && mb > 256.0);
   }
   if (!streams) a.nt = 0;
+  // the D3Q27 collisions bound by issue gain nothing on rows of whole sectors (fp32 MRT 64^3
+  // with far field 12.8 non-temporal, 13.8 us ordinary) and much on others (200 x 200 x 250
+  // 600 -> 428 us, fp16 160 x 180 x 193 BGK 198 -> 155 us)
+  if (L::Q == 27 && !op && COLL != COLL_GEIER_UNIT && COLL != TLBM_COLL_BGK && row % 32 == 0) a.nt = 1;
   a.rev = (rev || !streams) && !a.nt && mb > kSweepMB;
   a.run = op || !streams || (!a.nt && row % 128 != 0);
 }
