@@ -1705,7 +1705,9 @@ __global__ void k_force_add(const double* acc, T* bx, T* by, T* bz) {
 
 // Sum and rescale of a whole lattice as `planes` runs of `len` contiguous values, run p
 // at (p / inner_n) * outer + (p % inner_n) * inner.  A workgroup takes pieces of
-// MASS_PIECE values, four neighbouring ones to a lane and eight loads in flight; runs
+// MASS_PIECE values, sixteen bytes of neighbours to a lane (eight of 16-bit values) and
+// eight loads in flight, sixteen of FP64 (two loads to four neighbouring FP64 values leave
+// every other sixteen bytes of a wave's lines to the second one: 200^3 774 -> 704 us); runs
 // start at any element, which global memory operations allow.  The per-cell forms (k_moment_sums: four
 // FP64 sums and two 64-bit divisions per cell; k_scale) took 58 and 44 us on
 // 96 x 96 x 193 fp32; these take 22 and 42 us.  The sum leaves one FP64 partial per
@@ -1717,32 +1719,41 @@ struct Runs {
   int64_t outer, inner, len;
   uint32_t planes, inner_n, pieces;  // pieces per run
 };
-// four values from an address aligned like one of them (at least two bytes)
+// neighbouring values from an address aligned like one of them (at least two bytes)
 template <typename T>
-struct Vec4 {
-  typedef T type __attribute__((ext_vector_type(4), aligned(sizeof(T) < 4 ? sizeof(T) : 4)));
+struct VecN {
+  static constexpr int N = sizeof(T) == 8 ? 2 : 4;
+  typedef T type __attribute__((ext_vector_type(N), aligned(sizeof(T) < 4 ? sizeof(T) : 4)));
 };
 
-// fn4(values, address) on groups of four, fn1(value, address) on the last values of a run
-template <int S, class F4, class F1>
-__device__ __forceinline__ void for_pieces(typename Store<S>::T* f, const Runs& r, const F4& fn4, const F1& fn1) {
+// fnv(values, group, address) on groups of N, fn1(value, address) on what is left of a run
+template <int S, class FV, class F1>
+__device__ __forceinline__ void for_pieces(typename Store<S>::T* f, const Runs& r, const FV& fnv, const F1& fn1) {
   using T = typename Store<S>::T;
-  using V = typename Vec4<T>::type;
+  using V = typename VecN<T>::type;
+  constexpr uint32_t N = VecN<T>::N, G = MASS_PIECE / (256 * N);
   const uint64_t units = uint64_t(r.planes) * r.pieces;
   for (uint64_t u = blockIdx.x; u < units; u += gridDim.x) {
     const uint32_t p = uint32_t(u / r.pieces), k = uint32_t(u % r.pieces);
     const int64_t at = int64_t(k) * MASS_PIECE;
     T* base = f + int64_t(p / r.inner_n) * r.outer + int64_t(p % r.inner_n) * r.inner + at;
     const int64_t left = r.len - at;
-    const uint32_t lane = threadIdx.x * 4;
+    const uint32_t lane = threadIdx.x * N;
     if (left >= MASS_PIECE) {
-      V v[8];
+      V v[G];
 #pragma unroll
-      for (uint32_t j = 0; j < 8; ++j) v[j] = *(global_ptr<const V>)(base + (lane + j * 1024));
+      for (uint32_t j = 0; j < G; ++j) v[j] = *(global_ptr<const V>)(base + (lane + j * 256 * N));
 #pragma unroll
-      for (uint32_t j = 0; j < 8; ++j) fn4(v[j], (global_ptr<V>)(base + (lane + j * 1024)));
+      for (uint32_t j = 0; j < G; ++j) fnv(v[j], j, (global_ptr<V>)(base + (lane + j * 256 * N)));
     } else {
-      for (int64_t i = threadIdx.x; i < left; i += 256) fn1(base[i], (global_ptr<T>)(base + i));
+      const uint32_t whole = uint32_t(left) / N * N;
+#pragma unroll 4
+      for (uint32_t i = lane; i < whole; i += 256 * N) {
+        const V v = *(global_ptr<const V>)(base + i);
+        fnv(v, 0, (global_ptr<V>)(base + i));
+      }
+      const uint32_t i = whole + threadIdx.x;
+      if (i < left) fn1(base[i], (global_ptr<T>)(base + i));
     }
   }
 }
@@ -1750,13 +1761,14 @@ __device__ __forceinline__ void for_pieces(typename Store<S>::T* f, const Runs& 
 template <class L, int S>
 __global__ __launch_bounds__(256) void k_mass_sum(const void* fv, Runs r, double* partial) {
   using T = typename Store<S>::T;
-  using V = typename Vec4<T>::type;
+  using V = typename VecN<T>::type;
+  constexpr int N = VecN<T>::N;
   double a[4] = {0.0, 0.0, 0.0, 0.0};
   for_pieces<S>(
       static_cast<T*>(const_cast<void*>(fv)), r,
-      [&](const V& v, global_ptr<V>) {
+      [&](const V& v, uint32_t j, global_ptr<V>) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) a[e] += double(Store<S>::template get<L>(v[e], 0));
+        for (int e = 0; e < N; ++e) a[(int(j) * N + e) % 4] += double(Store<S>::template get<L>(v[e], 0));
       },
       [&](T v, global_ptr<T>) { a[0] += double(Store<S>::template get<L>(v, 0)); });
   const double s = wave_sum((a[0] + a[1]) + (a[2] + a[3]));
@@ -1779,12 +1791,12 @@ __global__ __launch_bounds__(256) void k_mass_scale(void* fv, Runs r, const doub
   __syncthreads();
   s = (part[0] + part[1]) + (part[2] + part[3]);
   const typename Store<S>::C scale = typename Store<S>::C(fabs(s) < 1e-30 ? 1.0 : target / s);
-  using V = typename Vec4<T>::type;
+  using V = typename VecN<T>::type;
   for_pieces<S>(
       static_cast<T*>(fv), r,
-      [&](V v, global_ptr<V> at) {
+      [&](V v, uint32_t, global_ptr<V> at) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = Store<S>::template put<L>(Store<S>::template get<L>(v[e], 0) * scale, 0);
+        for (int e = 0; e < VecN<T>::N; ++e) v[e] = Store<S>::template put<L>(Store<S>::template get<L>(v[e], 0) * scale, 0);
         *at = v;
       },
       [&](T v, global_ptr<T> at) { *at = Store<S>::template put<L>(Store<S>::template get<L>(v, 0) * scale, 0); });
