@@ -83,3 +83,23 @@ def test_fill_under_a_tangent(device, monkeypatch):
         c.fill_equilibrium()
         d = fw.unpack_dual(c.cavity(0))
         assert torch.equal(d.primal, w.expand_as(d.primal)) and not d.tangent.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,deviation", [(torch.float32, False), (torch.float64, False), (torch.float16, True),
+                                             (torch.bfloat16, True)])
+@pytest.mark.parametrize("shift", [0, 1, 2])
+def test_fill_writes_the_cells_and_nothing_else(dtype, deviation, shift):
+    """Edges whose planes are and are not whole sixteen-byte groups, buffers that do and do not start at one."""
+    edges = [3, 4, 5, 8, 31, 64, 66, 91]
+    c = tl.BatchedCavities(edges, [0.7] * len(edges), dtype=dtype, deviation=deviation)
+    buf = torch.full((c.a.numel() + shift + 8,), 7.0, dtype=dtype, device="cuda:0")
+    a = buf[shift:shift + c.a.numel()]
+    nat.check(nat.lib().tlbm_cavities_fill(c._store, a.data_ptr(), a.numel(), c._table, c.n, nat.stream_of(a)), "fill")
+    want = torch.full_like(buf, 7.0)
+    w = tl.lattice.D3Q19.W_EXACT64.to("cuda:0").reshape(19, 1, 1, 1)
+    for i, e in enumerate(edges):
+        p = (e * e + 63) // 64 * 64
+        v = want.as_strided((19, e, e, e), (p, 19 * p, e, 1), shift + c.offset(i))
+        v.copy_((torch.zeros_like(w) if deviation else w).expand_as(v))
+    assert torch.equal(buf, want)
