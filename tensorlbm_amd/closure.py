@@ -197,15 +197,18 @@ class _Adam:
         self.v = torch.zeros_like(self.m)
         self.t = 0
         self.bb = sizes()["batch_block"]
-        self.partials = torch.empty(((max_batch + self.bb - 1) // self.bb, model.nparam + 1), dtype=torch.float32,
-                                    device=model.device)
+        self.max_blocks = (max_batch + self.bb - 1) // self.bb
+        self.partials: torch.Tensor | None = None  # the workspace of step(); epoch() has its own
         self.loss = torch.zeros(1, dtype=torch.float32, device=model.device)
 
     def step(self, x: torch.Tensor, t: torch.Tensor) -> torch.Tensor:
         n = int(x.shape[0])
         nblk = (n + self.bb - 1) // self.bb
-        if nblk > self.partials.shape[0]:
+        if nblk > self.max_blocks:
             raise ValueError(f"minibatch of {n} exceeds the optimiser's buffer")
+        if self.partials is None:
+            self.partials = torch.empty((self.max_blocks, self.model.nparam + 1), dtype=torch.float32,
+                                        device=self.model.device)
         self.t += 1
         lib, s, p = nat.lib(), nat.stream_of(x), self.model.params.data_ptr()
         nat.check(lib.tlbm_mlp_grad(p, x.data_ptr(), t.data_ptr(), n, self.partials.data_ptr(), s), "tlbm_mlp_grad")
