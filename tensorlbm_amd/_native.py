@@ -241,37 +241,43 @@ def stream_of(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+# bound once, without torch's Python wrappers: an obstacle loop on a small grid asks twice a step and waits for the host
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+_is_tracing, _len_dispatch, _len_function = (
+    torch._C._is_tracing, torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack)
+_transform = torch._C._functorch.peek_interpreter_stack
+_is_compiling, _inference_mode = torch.compiler.is_compiling, torch.is_inference_mode_enabled
+_increment_version = torch.autograd.graph.increment_version
+
+
 def on_current_device(t: torch.Tensor) -> bool:
     """Whether launches on torch's current stream of the tensor's device reach that device."""
-    return t.get_device() == torch.cuda.current_device()
+    return t.get_device() == _current_device()
 
 
 def eager_write(*tensors: torch.Tensor) -> bool:
     """Whether a kernel may read and write these tensors by address in place of torch's in-place operators:
     plain tensors on the current device, with no gradient, tangent or transform (vmap, grad, functionalize) on
     them and no dispatch or function mode, tracer or compiler watching; inference tensors only in inference mode."""
-    if torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() or \
-            torch.compiler.is_compiling() or torch.jit.is_tracing():
+    if _is_compiling() or _is_tracing() or _len_dispatch() or _transform() is not None:
         return False
-    if torch._C._len_torch_function_stack() and not all(
-            isinstance(m, DeviceContext) for m in _get_current_function_mode_stack()):
+    if _len_function() and not all(isinstance(m, DeviceContext) for m in _get_current_function_mode_stack()):
         return False
+    device = tensors[0].get_device()
     for t in tensors:
-        if type(t) is not torch.Tensor or t.requires_grad or t.is_neg() or not on_current_device(t):
+        if type(t) is not torch.Tensor or t.requires_grad or t.is_neg() or t.get_device() != device:
             return False
-        if t.is_inference() and not torch.is_inference_mode_enabled():
+        if t.is_inference() and not _inference_mode():
             return False
         if forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None:
             return False
-    return True
+    return on_current_device(tensors[0])
 
 
 def written(*tensors: torch.Tensor) -> None:
     """Tell autograd of a kernel's write, as an in-place operator does, so that a backward pass that saved one of
-    these tensors raises instead of using the new values."""
-    for t in tensors:
-        if not t.is_inference():
-            torch.autograd.graph.increment_version(t)
+    these tensors raises instead of using the new values (inference tensors have no version and stay as they are)."""
+    _increment_version(tensors)
 
 
 def require_gpu(t: torch.Tensor, what: str) -> None:

@@ -218,8 +218,9 @@ def fused_obstacle_step(
     _launch_step(f, out, coll, solid=solid, force=acc, what="fused_obstacle_step")
     if force is None and acc is not None:
         dt = fx_buf.dtype
-        if dt in (torch.float32, torch.float64) and all(
-                b.numel() == 1 and b.dtype == dt and b.device == f.device for b in bufs) and nat.eager_write(*bufs):
+        if dt in (torch.float32, torch.float64) and fx_buf.get_device() == f.get_device() and \
+                fy_buf.dtype == dt and fz_buf.dtype == dt and \
+                fx_buf.numel() == fy_buf.numel() == fz_buf.numel() == 1 and nat.eager_write(*bufs):
             nat.check(nat.lib().tlbm_force_add(nat.store_code(dt), acc.data_ptr(), *(b.data_ptr() for b in bufs),
                                                nat.stream_of(f)), "fused_obstacle_step")
             nat.written(*bufs)
@@ -233,6 +234,8 @@ def _distinct(f: torch.Tensor) -> bool:
     """No two elements of ``f`` share memory and x is its fastest axis (stride 1)."""
     if f.stride(-1) != 1:
         return False
+    if f.is_contiguous():
+        return f.numel() > 0
     span = 1
     for n, st in sorted(((n, st) for n, st in zip(f.shape, f.stride()) if n > 1), key=lambda v: v[1]):
         if st < span:
