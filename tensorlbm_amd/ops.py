@@ -131,8 +131,9 @@ def _new_like(f):
 def _macroscopic(f, q, what):
     f, dims = _pops(f, q, what)
     dt = _eager_dtype(f, what)
-    rho, ux, uy = (_new_like(f[0]) for _ in range(3))
-    uz = _new_like(f[0]) if q != 9 else None
+    rho = _new_like(f[0])
+    ux, uy = torch.empty_like(rho), torch.empty_like(rho)
+    uz = torch.empty_like(rho) if q != 9 else None
     rc = nat.lib().tlbm_macroscopic(q, dt, f.data_ptr(), rho.data_ptr(), ux.data_ptr(), uy.data_ptr(),
                                     nat.ptr(uz), dims[0] * dims[1] * dims[2], nat.stream_of(f))
     nat.check(rc, what)
