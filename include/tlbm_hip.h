@@ -432,7 +432,7 @@ typedef struct tlbm_cavity {
 int tlbm_cavities_layout(tlbm_cavity* cavs, int n, int64_t* total_elements, int64_t* total_tiles);
 
 /* tlbm_cavities_fill: every cavity at rest, rho = 1 (f_q = w_q; 0 in deviation storage), the padding
- * untouched.
+ * untouched; the cavities' tau may be anything.
  * tlbm_cavities_step: one step of every cavity, f_in -> f_out (distinct buffers of `capacity` elements; store
  * F32, F64, F16_DEV or BF16_DEV).  grid = 0: one workgroup per tile; grid > 0: a persistent
  * grid of that many workgroups striding over the tiles. */

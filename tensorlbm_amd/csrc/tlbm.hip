@@ -978,9 +978,10 @@ __global__ __launch_bounds__(256) void k_lbm(const KArgs<typename Store<S>::C> a
 // The base tile's kernel is built with its shape at compile time beside the run-time form:
 // in the run-time form the index arithmetic of the pulls costs instructions and, with the
 // state of the force sample, registers.  Base tile, run-time / compile-time shape, us per
-// launch: fp32 MRT with force 256^3 767 / 595, 128^3 102 / 87; BGK with force 256^3 514 /
-// 485, without 482 / 464; fp16-deviation BGK channel 256^3 453 / 439; fp32 cumulant channel
-// 64^3 18.3 / 17.2; D3Q27 MRT 256^3 1074 / 1042.
+// launch (medians over five placements of the buffers): fp32 MRT with force 256^3 769 / 603,
+// 128^3 102 / 88; BGK with force 256^3 513 / 497, without 486 / 485; fp16-deviation BGK
+// channel 256^3 453 / 442; fp32 cumulant channel 64^3 18.3 / 17.4; D3Q27 MRT 256^3
+// 1078 / 1040.
 template <class L, int S, int COLL, int FEAT, int BCK, Tile2 Tile>
 __global__ __launch_bounds__((tile2_threads<L, S>())) void k_lbm2(const KArgs<typename Store<S>::C> a,
                                                                   const Plan2 p2) {
@@ -1340,7 +1341,7 @@ __global__ __launch_bounds__(256) void k_equilibrium(const T* rho, const T* ux, 
 // `order` (macro_order): 1 runs of workgroups per XCD, 2 these from the last cells on, which of
 // a lattice somewhat larger than the memory-side cache are the ones still in it (128^3 fp64
 // after a boundary op: 92 -> 74 us); 0 as they come: with nothing left in the cache the runs
-// cost (fp32 256^3 290 against 272 us, D2Q9 fp32 6144^2 324 against 296).
+// cost (fp32 256^3 303 against 274 us, D2Q9 fp32 6144^2 342 against 298).
 template <class L, typename T>
 __global__ __launch_bounds__(256) void k_macroscopic(const T* f, T* rho, T* ux, T* uy, T* uz, uint64_t N,
                                                      int order) {
@@ -1659,7 +1660,7 @@ __global__ __launch_bounds__(256) void k_scale(void* fv, Layout lay, const doubl
 // edges, so every cell is written once with the value the last of them leaves.  The
 // outlet reads x = nx-2, which no face of its row writes (nx = 2: the inlet's value).
 // One launch instead of a plane copy per face and the small operators that built the
-// face value: 96 x 96 x 193 fp32, about 25 launches -> one of 11.6 us.  Lanes enumerate a
+// face value: 96 x 96 x 193 fp32, about 25 launches -> one of 11.4 us.  Lanes enumerate a
 // population's face cells: first the (z, y) pairs of the x faces, whose two cells lie
 // next to each other in memory (x = nx-1 of a row, x = 0 of the next), then the rows
 // of the y faces and the z planes, contiguous.  blockIdx.y: population.
@@ -1707,10 +1708,10 @@ __global__ void k_force_add(const double* acc, T* bx, T* by, T* bz) {
 // at (p / inner_n) * outer + (p % inner_n) * inner.  A workgroup takes pieces of
 // MASS_PIECE values, sixteen bytes of neighbours to a lane (eight of 16-bit values) and
 // eight loads in flight, sixteen of FP64 (two loads to four neighbouring FP64 values leave
-// every other sixteen bytes of a wave's lines to the second one: 200^3 774 -> 704 us); runs
+// every other sixteen bytes of a wave's lines to the second one: 200^3 780 -> 699 us); runs
 // start at any element, which global memory operations allow.  The per-cell forms (k_moment_sums: four
 // FP64 sums and two 64-bit divisions per cell; k_scale) took 58 and 44 us on
-// 96 x 96 x 193 fp32; these take 22 and 42 us.  The sum leaves one FP64 partial per
+// 96 x 96 x 193 fp32; these take 21 and 42 us.  The sum leaves one FP64 partial per
 // workgroup, added up in a fixed order by every workgroup of the scaling, so there is
 // no atomic, nothing to clear and the result does not vary from run to run.
 constexpr int MASS_PIECE = 256 * 4 * 8;
@@ -2513,9 +2514,9 @@ constexpr double kSweepMB = 145.0;
 // output, which one more op reads, the other way round above kSweepMB.  Above kOpsMB nothing
 // of one op's output is left for the next, and on rows of whole lines the ops do better with
 // non-temporal stores, ordinary loads and the plain order.  Caches and runs against that, us
-// for collide and for collide and stream in turn: fp32 256^3 474 and 1033 against 448 and 886,
-// D3Q27 fp32 128 x 128 x 256 (453 MB) 176 and 347 against 164 and 320, fp64 256^3 931 and 1870
-// against 896 and 1804, D2Q9 fp32 4096^2 212 and 433 against 203 and 403; at 319 MB 109 and 219
+// for collide and for collide and stream in turn: fp32 256^3 472 and 1070 against 449 and 893,
+// D3Q27 fp32 128 x 128 x 256 (453 MB) 180 and 333 against 164 and 324, fp64 256^3 946 and 1875
+// against 900 and 1839, D2Q9 fp32 4096^2 210 and 420 against 203 and 406; at 319 MB 109 and 219
 // against 121 and 237.  Rows of partial lines keep them: fp32 200^3 233 and 448 against 311 and
 // 602.
 constexpr double kOpsMB = 330.0;
@@ -2540,8 +2541,8 @@ void set_sweep(KArgs<C>& a, bool streams, bool rev) {
   }
   if (!streams) a.nt = 0;
   // the D3Q27 collisions bound by issue gain nothing on rows of whole sectors (fp32 MRT 64^3
-  // with far field 12.8 non-temporal, 13.8 us ordinary) and much on others (200 x 200 x 250
-  // 600 -> 428 us, fp16 160 x 180 x 193 BGK 198 -> 155 us)
+  // with far field 13.0 non-temporal, 13.8 us ordinary) and much on others (200 x 200 x 250
+  // 618 -> 430 us, fp16 160 x 180 x 193 BGK 203 -> 154 us)
   if (L::Q == 27 && !op && COLL != COLL_GEIER_UNIT && COLL != TLBM_COLL_BGK && row % 32 == 0) a.nt = 1;
   a.rev = (rev || !streams) && !a.nt && mb > kSweepMB;
   a.run = op || !streams || (!a.nt && row % 128 != 0);
